@@ -235,31 +235,39 @@ struct NodalGlobal
   __device__ __forceinline__ double operator()(int n) const { return v[nid[n]]; }
 };
 
-// The K+ parameters of one node at one quadrature point of an Euler cell.
-// With the acoustic pairs written as
-//   r+- = (rho / 2a) (r0 +- a e_n),  l+- = (l0v +- a f_n) / (rho a),
-//   r0 = (1, V, H), e_n = (0, n, V.n), l0v = (gm1 |V|^2 / 2, -gm1 V, gm1),
-//   f_n = (-V.n, n, 0),
-// K+_n = l0_n I + dp_n r+ l+^T + dm_n r- l-^T becomes
-//   K+_n x = l0_n x + alpha r0 + beta e_n,
-//   alpha = (sg_n P + a dl_n Q) / 2a^2, beta = sg_n Q / 2 + dl_n P / 2a,
-//   P = l0v . x, Q = f_n . x, sg = dp + dm, dl = dp - dm,
-// and S = sum_n K+_n needs only sum l0, sum sg, w = sum dl n and
-// T = sum sg n n^T. nh = g / |g| for the physical gradient g of the node's
-// basis function, um = V . nh, emax the largest |eigenvalue| |g| (um, um +- a).
+// K+ of the Euler cells in the variables that block-diagonalise it. At a point
+// with velocity V, total enthalpy H and sound speed a, a vector x has the parts
+//   p = (gm1 / a) (|V|^2/2 x_0 - V . x_m + x_E),  Q = x_m - V x_0,  s = x_0 - p / a,
+//   x = s (1, V, |V|^2/2) + (p / a) (1, V, H) + (0, Q, V . Q),
+// and the upwind matrix of a node with unit gradient n acts on them as
+//   s -> l0 s,  p -> l0 p + al,  Q -> l0 Q + be n,
+//   al = hs p + hd (n . Q),  be = hs (n . Q) + hd p,
+// l0, lp, lm the positive parts of |g| (V.n), |g| (V.n + a), |g| (V.n - a),
+// hs = (lp + lm) / 2 - l0, hd = (lp - lm) / 2; in conservative variables
+//   K+_n x = l0 x + (al / a) (1, V, H) + be (0, n, V . n).
+// So S = sum_n K+_n is sum l0 on s and, on (p, Q), the symmetric positive
+// definite (D + 1) x (D + 1) matrix
+//   [ sum l0 + sum hs, w^T; w, sum l0 I + T ],  w = sum hd n, T = sum hs n n^T,
+// whose solve needs no pivoting: one reciprocal and a Cholesky-like
+// elimination of 3 (2D) or 4 (3D) unknowns instead of the elimination with row
+// swaps of a 4 x 4 or 5 x 5 matrix, whose selects alone were a hundred (2D) to
+// 240 (3D) instructions of a quadrature point. These cells are bound by FP64
+// issue and latency, so a sweep follows the count: 786 432 P2 / Q2 cells (LDA)
+// 368 -> 301 us, 5.3 M P1 tetrahedra (PSI / LDA blend) 1.86 -> 1.44 ms, 0.66 M
+// P2 tetrahedra (LDA) 605 -> 516 us, with 40 to 150 registers less.
 template <int D>
 struct EulerNodeK
 {
-  double l0, sg, dl, um, nh[D], emax;
+  double l0, hs, hd, un, nh[D], emax;
 };
 
 // The geometric part of a node's K+ parameters: nh = g / |g| and |g| for the
-// physical gradient g of the node's basis function (tiny: |g| negligible).
+// physical gradient g of the node's basis function; normk: |g|, or 0 where
+// |g| is negligible (and nh = 0 then).
 template <int D>
 struct EulerNodeG
 {
-  double nh[D], norm;
-  bool tiny;
+  double nh[D], norm, normk;
 };
 
 // Jq: the inverse Jacobian at the point, dvk: the reference gradients of the
@@ -282,37 +290,34 @@ __device__ __forceinline__ EulerNodeG<D> euler_node_g(const double (&Jq)[D][D], 
   double norm, inorm;
   sqrt_rsqrt(nn, norm, inorm);
   norm = (nn > 0.0) ? norm : 0.0;  // sqrt_rsqrt(0) is NaN
-  ge.tiny = (D == 2) ? (norm < 1.e-9) : (norm == 0.0);
-  inorm = ge.tiny ? 0.0 : inorm;
+  const bool tiny = (D == 2) ? (norm < 1.e-9) : (norm == 0.0);
+  inorm = tiny ? 0.0 : inorm;
 #pragma unroll
   for (int x = 0; x < D; ++x) ge.nh[x] = g[x] * inorm;
   ge.norm = norm;
+  ge.normk = (D == 2) ? (tiny ? 0.0 : norm) : norm;
   return ge;
 }
 
 // The K+ parameters from the geometric part and the point's velocity V and
-// sound speed a.
+// sound speed a; un = V . nh, emax the largest |eigenvalue| |g| (un, un +- a).
 template <int D>
 __device__ __forceinline__ EulerNodeK<D> euler_node_k(const EulerNodeG<D> &ge, const double (&V)[D], double a)
 {
   EulerNodeK<D> k;
-  double u_n = 0.0;
+  double un = 0.0;
 #pragma unroll
   for (int x = 0; x < D; ++x) {
     k.nh[x] = ge.nh[x];
-    u_n += V[x] * k.nh[x];
+    un += V[x] * ge.nh[x];
   }
-  k.um = u_n;
-  const double norm = ge.norm;
-  const bool tiny = ge.tiny;
-  const double e0 = norm * u_n, ep = norm * (u_n + a), em = norm * (u_n - a);
-  k.emax = fmax(fabs(e0), fmax(fabs(ep), fabs(em)));
-  const double p0 = fmax(0.0, e0);
-  const double dpn = tiny ? 0.0 : fmax(0.0, ep) - p0;
-  const double dmn = tiny ? 0.0 : fmax(0.0, em) - p0;
-  k.l0 = tiny ? 0.0 : p0;
-  k.sg = dpn + dmn;
-  k.dl = dpn - dmn;
+  k.un = un;
+  const double e0 = ge.norm * un, c = ge.normk * a;
+  k.emax = fabs(e0) + ((D == 2) ? ge.norm * a : c);
+  k.l0 = fmax(0.0, e0);
+  const double lp = fmax(0.0, e0 + c), lm = fmax(0.0, e0 - c);
+  k.hs = 0.5 * (lp + lm) - k.l0;
+  k.hd = 0.5 * (lp - lm);
   return k;
 }
 
@@ -323,79 +328,198 @@ __device__ __forceinline__ EulerNodeK<D> euler_node_k(const double (&Jq)[D][D], 
   return euler_node_k<D>(euler_node_g<D, ND>(Jq, dvk, n), V, a);
 }
 
-// out = K+_n v at a point with velocity V, total enthalpy H, sound speed a,
-// i2a = 1 / 2a, i2a2 = 1 / 2a^2 and l0v as above.
+// A point's quantities in those variables (hv = |V|^2 / 2, ga = gm1 / a).
 template <int D>
-__device__ __forceinline__ void euler_kplus(const EulerNodeK<D> &k, const double (&l0v)[D + 2], const double (&V)[D],
-                                            double H, double a, double i2a, double i2a2, const double (&v)[D + 2],
-                                            double (&out)[D + 2])
+struct EulerPoint
 {
-  constexpr int M = D + 2;
-  double P = 0.0;
+  double V[D], H, a, ia, hv, ga;
+  __device__ __forceinline__ double p_of(const double (&x)[D + 2]) const
+  {
+    double t = x[D + 1] + hv * x[0];
 #pragma unroll
-  for (int c = 0; c < M; ++c) P += l0v[c] * v[c];
-  double Q = -k.um * v[0];
+    for (int d = 0; d < D; ++d) t -= V[d] * x[1 + d];
+    return ga * t;
+  }
+  // K+ of a node from (p, n . Q) of a vector: al / a and be
+  __device__ __forceinline__ void acoustic(const EulerNodeK<D> &k, double p, double t, double &al, double &be) const
+  {
+    al = (k.hs * p + k.hd * t) * ia;
+    be = k.hs * t + k.hd * p;
+  }
+  // out += l0 x + al (1, V, H) + be (0, n, V . n)
+  __device__ __forceinline__ void add(const EulerNodeK<D> &k, const double (&x)[D + 2], double al, double be,
+                                      double (&out)[D + 2]) const
+  {
+    out[0] += k.l0 * x[0] + al;
 #pragma unroll
-  for (int x = 0; x < D; ++x) Q += k.nh[x] * v[1 + x];
-  const double al = (k.sg * P + a * k.dl * Q) * i2a2;
-  const double be = 0.5 * k.sg * Q + k.dl * P * i2a;
-  out[0] = k.l0 * v[0] + al;
+    for (int d = 0; d < D; ++d) {
+      double t = out[1 + d] + k.l0 * x[1 + d];
+      t += al * V[d];
+      out[1 + d] = t + be * k.nh[d];
+    }
+    double t = out[D + 1] + k.l0 * x[D + 1];
+    t += al * H;
+    out[D + 1] = t + be * k.un;
+  }
+  // out += K+ x with (p, Q) of x at hand, or from x itself
+  __device__ __forceinline__ void apply(const EulerNodeK<D> &k, const double (&x)[D + 2], double p,
+                                        const double (&Q)[D], double (&out)[D + 2]) const
+  {
+    double t = 0.0, al, be;
 #pragma unroll
-  for (int x = 0; x < D; ++x) out[1 + x] = k.l0 * v[1 + x] + al * V[x] + be * k.nh[x];
-  out[M - 1] = k.l0 * v[M - 1] + al * H + be * k.um;
+    for (int d = 0; d < D; ++d) t += k.nh[d] * Q[d];
+    acoustic(k, p, t, al, be);
+    add(k, x, al, be, out);
+  }
+  __device__ __forceinline__ void apply(const EulerNodeK<D> &k, const double (&x)[D + 2], double (&out)[D + 2]) const
+  {
+    double t = -k.un * x[0], al, be;
+#pragma unroll
+    for (int d = 0; d < D; ++d) t += k.nh[d] * x[1 + d];
+    acoustic(k, p_of(x), t, al, be);
+    add(k, x, al, be, out);
+  }
+};
+
+// S = sum_n K+_n: the sums over the nodes, then the factors of its solve.
+template <int D>
+struct EulerSum
+{
+  double l0, hs, w[D], T[D][D];
+  double il0, ip[D + 1], L[D + 1][D + 1];
+  __device__ __forceinline__ void clear()
+  {
+    l0 = hs = 0.0;
+#pragma unroll
+    for (int x = 0; x < D; ++x) {
+      w[x] = 0.0;
+#pragma unroll
+      for (int y = x; y < D; ++y) T[x][y] = 0.0;
+    }
+  }
+  __device__ __forceinline__ void add(const EulerNodeK<D> &k)
+  {
+    l0 += k.l0;
+    hs += k.hs;
+#pragma unroll
+    for (int x = 0; x < D; ++x) {
+      w[x] += k.hd * k.nh[x];
+      const double t = k.hs * k.nh[x];
+#pragma unroll
+      for (int y = x; y < D; ++y) T[x][y] += t * k.nh[y];
+    }
+  }
+  // L D L^T of the (p, Q) block
+  __device__ __forceinline__ void factor()
+  {
+    constexpr int K = D + 1;
+    double A[K][K];
+    A[0][0] = l0 + hs;
+#pragma unroll
+    for (int x = 0; x < D; ++x) {
+      A[0][1 + x] = w[x];
+#pragma unroll
+      for (int y = x; y < D; ++y) A[1 + x][1 + y] = T[x][y] + ((x == y) ? l0 : 0.0);
+    }
+    il0 = recip(l0);
+#pragma unroll
+    for (int c = 0; c < K; ++c) {
+      ip[c] = recip(A[c][c]);
+#pragma unroll
+      for (int r = c + 1; r < K; ++r) {
+        const double f = A[c][r] * ip[c];
+        L[r][c] = f;
+#pragma unroll
+        for (int j = r; j < K; ++j) A[r][j] -= f * A[c][j];
+      }
+    }
+  }
+  // x = S^-1 b in conservative variables, with its (p, Q)
+  __device__ __forceinline__ void solve(const EulerPoint<D> &pt, const double (&b)[D + 2], double (&x)[D + 2],
+                                        double &p, double (&Q)[D]) const
+  {
+    constexpr int K = D + 1;
+    double y[K];
+    y[0] = pt.p_of(b);
+    const double s = (b[0] - y[0] * pt.ia) * il0;
+#pragma unroll
+    for (int d = 0; d < D; ++d) y[1 + d] = b[1 + d] - pt.V[d] * b[0];
+#pragma unroll
+    for (int r = 1; r < K; ++r)
+#pragma unroll
+      for (int c = 0; c < r; ++c) y[r] -= L[r][c] * y[c];
+#pragma unroll
+    for (int r = K - 1; r >= 0; --r) {
+      double t = y[r] * ip[r];
+#pragma unroll
+      for (int c = r + 1; c < K; ++c) t -= L[c][r] * y[c];
+      y[r] = t;
+    }
+    p = y[0];
+    const double pa = p * pt.ia;
+    x[0] = s + pa;
+    double e = s * pt.hv + pa * pt.H;
+#pragma unroll
+    for (int d = 0; d < D; ++d) {
+      Q[d] = y[1 + d];
+      x[1 + d] = pt.V[d] * x[0] + Q[d];
+      e += pt.V[d] * Q[d];
+    }
+    x[D + 1] = e;
+  }
+};
+
+template <int D>
+__device__ __forceinline__ EulerPoint<D> euler_point(const EulerState<double, D> &st, double gm1)
+{
+  EulerPoint<D> pt;
+#pragma unroll
+  for (int d = 0; d < D; ++d) pt.V[d] = st.V[d];
+  pt.H = st.H;
+  pt.a = st.a;
+  pt.ia = st.inv_a;
+  pt.hv = 0.5 * st.v2;
+  pt.ga = gm1 * st.inv_a;
+  return pt;
 }
 
-// S = sum_n K+_n from the node sums (sl0 = sum l0, ssg = sum sg, w, T) as
-// S = sl0 I + ssg/2a^2 r0 l0v^T + 1/2 sum sg e f^T + 1/2a (r0 (F w)^T + (E w) l0v^T).
+// sum_n K+_n U_n over the nodes of a point, gathered in parts: sum l0 U, sum
+// al / a, sum be n and sum be (V . n).
 template <int D>
-__device__ __forceinline__ void euler_kplus_sum(double sl0, double ssg, const double (&w)[D], const double (&T)[D][D],
-                                                const double (&l0v)[D + 2], const double (&V)[D], double H,
-                                                double i2a, double i2a2, double (&A)[D + 2][D + 2])
+struct EulerKU
 {
-  constexpr int M = D + 2;
-  double r0[M], ew[M], fw[M];
-  r0[0] = 1.0;
+  double lu[D + 2], al, be[D], bu;
+  __device__ __forceinline__ void clear()
+  {
 #pragma unroll
-  for (int x = 0; x < D; ++x) r0[1 + x] = V[x];
-  r0[M - 1] = H;
-  double vw = 0.0;
+    for (int k = 0; k < D + 2; ++k) lu[k] = 0.0;
+    al = bu = 0.0;
 #pragma unroll
-  for (int x = 0; x < D; ++x) vw += V[x] * w[x];
-  ew[0] = 0.0;
-  fw[0] = -vw;
-#pragma unroll
-  for (int x = 0; x < D; ++x) {
-    ew[1 + x] = w[x];
-    fw[1 + x] = w[x];
+    for (int d = 0; d < D; ++d) be[d] = 0.0;
   }
-  ew[M - 1] = vw;
-  fw[M - 1] = 0.0;
-  double TV[D], VTV = 0.0;
+  __device__ __forceinline__ void add(const EulerPoint<D> &pt, const EulerNodeK<D> &k, const double (&x)[D + 2])
+  {
+    double t = -k.un * x[0];
 #pragma unroll
-  for (int x = 0; x < D; ++x) {
-    double t = 0.0;
+    for (int d = 0; d < D; ++d) t += k.nh[d] * x[1 + d];
+    const double p = pt.p_of(x);
+    al += k.hs * p + k.hd * t;
+    const double b = k.hs * t + k.hd * p;
 #pragma unroll
-    for (int y = 0; y < D; ++y) t += T[x][y] * V[y];
-    TV[x] = t;
-    VTV += V[x] * t;
+    for (int d = 0; d < D; ++d) be[d] += b * k.nh[d];
+    bu += b * k.un;
+#pragma unroll
+    for (int c = 0; c < D + 2; ++c) lu[c] += k.l0 * x[c];
   }
-  const double c1 = ssg * i2a2;
+  __device__ __forceinline__ void total(const EulerPoint<D> &pt, double (&out)[D + 2]) const
+  {
+    const double ai = al * pt.ia;
+    out[0] = lu[0] + ai;
 #pragma unroll
-  for (int i = 0; i < M; ++i)
-#pragma unroll
-    for (int j = 0; j < M; ++j) {
-      // 1/2 sum_n sg_n e_n f_n^T
-      double et = 0.0;
-      if (i >= 1 && i <= D) {
-        if (j == 0) et = -TV[i - 1];
-        else if (j <= D) et = T[i - 1][j - 1];
-      } else if (i == M - 1) {
-        if (j == 0) et = -VTV;
-        else if (j <= D) et = TV[j - 1];
-      }
-      A[i][j] = ((i == j) ? sl0 : 0.0) + c1 * r0[i] * l0v[j] + 0.5 * et + i2a * (r0[i] * fw[j] + ew[i] * l0v[j]);
-    }
-}
+    for (int d = 0; d < D; ++d) out[1 + d] = lu[1 + d] + ai * pt.V[d] + be[d];
+    out[D + 1] = lu[D + 1] + ai * pt.H + bu;
+  }
+};
 
 // Residuals phi[ND][M] and wave speed of one element from its vertex
 // coordinates X and nodal state U. lds_div: this thread's slice of NQ*M
@@ -541,9 +665,13 @@ __device__ __forceinline__ void cell_residual(const double *__restrict__ tab, co
   }
 
   // ---- element scheme ------------------------------------------------------
+  // NDIS: the scheme has the N dissipation. B and the PSI / LDA blend need it
+  // apart from the LDA part (DIS2); N and PSI only their sum, which one K+
+  // product per node and point gives: K+_n (w U_n + y), S y = w (r - sum K+ U).
   constexpr bool NDIS = (SC != SC_LDA);
-  double lda[ND][M];
-  double dis[NDIS ? ND : 1][M];
+  constexpr bool DIS2 = (SC == SC_B || SC == SC_BPSI);
+  double lda[ND][M];  // (N and PSI: the N residual)
+  double dis[DIS2 ? ND : 1][M];
   // max over nodes and quadrature points of |eigenvalue|; the floor 1e-6 of
   // every (node, point) term is applied once at the end (max(1e-6, max x) =
   // max over x of max(1e-6, x))
@@ -555,25 +683,25 @@ __device__ __forceinline__ void cell_residual(const double *__restrict__ tab, co
     for (int k = 0; k < M; ++k) lda[n][k] = 0.0;
   }
 #pragma unroll
-  for (int n = 0; n < (NDIS ? ND : 1); ++n)
+  for (int n = 0; n < (DIS2 ? ND : 1); ++n)
 #pragma unroll
     for (int k = 0; k < M; ++k) dis[n][k] = 0.0;
 #pragma unroll
   for (int k = 0; k < M; ++k) fint[k] = 0.0;
   double vol = 0.0;
 
-  // TWO: the dissipative schemes of the 3D P2 cells (affine, NQ 3 M <= ND (M
-  // + 1)) in two passes over the quadrature points, so that neither holds the
-  // K+ parameters of all nodes beside the 2 ND M residual sums:
+  // TWO: the dissipative schemes of the 3D P2 cells (affine, NQ (1 + R) M <=
+  // ND (M + 1), R right-hand sides) in two passes over the quadrature points,
+  // so that neither holds the K+ parameters of all nodes beside the residual
+  // sums:
   //   1. per point q: S_q = sum_n K+_n (one evaluation of each node's
-  //      parameters, which also gives sum_n K+_n U_n), the solve for the LDA
-  //      weights x_q = w_q S_q^-1 r_q and ub_q = S_q^-1 sum_n K+_n U_n; the
+  //      parameters, which also gives sum_n K+_n U_n) and its solves; the
   //      point's (V, a, H) replace its divergence slice in the LDS column and
-  //      x_q, w_q ub_q follow the slices;
-  //   2. per point q again, every node: K+_n x_q and K+_n (w_q U_n - w_q ub_q)
-  //      added to the node's LDA and dissipation sums (a second evaluation of
-  //      the parameters).
-  constexpr bool TWO = (D == 3) && NDIS && AFFINE && DLDS && (M == D + 2) && (NQ * 3 * M <= ND * (M + 1));
+  //      the R solutions follow the slices;
+  //   2. per point q again, every node: its K+ products added to its sums (a
+  //      second evaluation of the parameters).
+  constexpr int R = DIS2 ? 2 : 1;
+  constexpr bool TWO = (D == 3) && NDIS && AFFINE && DLDS && (M == D + 2) && (NQ * (1 + R) * M <= ND * (M + 1));
 
   // P1 simplices of the Euler physics (affine, D + 1 nodes): the basis
   // gradients, and with them the geometric part of every node's K+
@@ -676,8 +804,9 @@ __device__ __forceinline__ void cell_residual(const double *__restrict__ tab, co
       const double wr = wj * inv * r[0];
 #pragma unroll
       for (int n = 0; n < ND; ++n) {
-        lda[n][0] += kp[n] * wr;
-        if constexpr (NDIS) dis[n][0] += wj * (kp[n] * (Uq(n, 0) - ub));
+        if constexpr (DIS2 || !NDIS) lda[n][0] += kp[n] * wr;
+        if constexpr (DIS2) dis[n][0] += wj * (kp[n] * (Uq(n, 0) - ub));
+        if constexpr (NDIS && !DIS2) lda[n][0] += kp[n] * (wr + wj * (Uq(n, 0) - ub));
       }
     } else {
       double uq[M];
@@ -690,52 +819,37 @@ __device__ __forceinline__ void cell_residual(const double *__restrict__ tab, co
       }
       const EulerState<double, D> st = euler_state<double, D>(uq, double(pp.p0));
       bad = bad || st.bad;
-      const double gm1 = pp.p0 - 1.0;
+      const EulerPoint<D> pt = euler_point<D>(st, pp.p0 - 1.0);
       const double *dvk = dvq;
-      // compact K+ of every node (EulerNodeK, euler_kplus)
       using NodeK = EulerNodeK<D>;
       // the K+ parameters of node n (recomputed where keeping them for all
       // nodes costs spills)
       auto node_k = [&](const int n) {
         if constexpr (CG)
-          return euler_node_k<D>(cg[n], st.V, st.a);
+          return euler_node_k<D>(cg[n], pt.V, pt.a);
         else
-          return euler_node_k<D, ND>(Jq, dvk, n, st.V, st.a);
+          return euler_node_k<D, ND>(Jq, dvk, n, pt.V, pt.a);
       };
       // 3D: recompute in the application instead of keeping ND sets
       constexpr bool KEEP = (D == 2);
       NodeK nk[KEEP ? ND : 1];
-      double sl0 = 0.0, ssg = 0.0, w[D], T[D][D];
-#pragma unroll
-      for (int x = 0; x < D; ++x) {
-        w[x] = 0.0;
-#pragma unroll
-        for (int y = 0; y < D; ++y) T[x][y] = 0.0;
-      }
+      EulerSum<D> S;
+      S.clear();
+      EulerKU<D> ku;
+      if constexpr (NDIS) ku.clear();
 #pragma unroll
       for (int n = 0; n < ND; ++n) {
         const NodeK k = node_k(n);
         if constexpr (KEEP) nk[n] = k;
         lmax = fmax(lmax, k.emax);
-        sl0 += k.l0;
-        ssg += k.sg;
+        S.add(k);
+        if constexpr (NDIS) {
+          double un[M];
 #pragma unroll
-        for (int x = 0; x < D; ++x) {
-          w[x] += k.dl * k.nh[x];
-#pragma unroll
-          for (int y = 0; y < D; ++y) T[x][y] += k.sg * k.nh[x] * k.nh[y];
+          for (int c = 0; c < M; ++c) un[c] = Uq(n, c);
+          ku.add(pt, k, un);
         }
       }
-      const double a = st.a;
-      const double i2a = 0.5 * st.inv_a, i2a2 = i2a * st.inv_a;
-      double l0v[M];
-      l0v[0] = 0.5 * gm1 * st.v2;
-#pragma unroll
-      for (int x = 0; x < D; ++x) l0v[1 + x] = -gm1 * st.V[x];
-      l0v[M - 1] = gm1;
-      auto kplus = [&](const NodeK &k, const double (&v)[M], double (&out)[M]) {
-        euler_kplus<D>(k, l0v, st.V, st.H, a, i2a, i2a2, v, out);
-      };
       auto node_at = [&](const int n) -> NodeK {
         if constexpr (KEEP) {
           return nk[n];
@@ -753,87 +867,24 @@ __device__ __forceinline__ void cell_residual(const double *__restrict__ tab, co
           return node_k(n);
         }
       };
-      // S as in euler_kplus_sum, written out here: the call changes the
-      // register allocation of the 2D quadrilateral cells (a 16-byte spill)
-      // S = sl0 I + ssg/2a^2 r0 l0v^T + 1/2 sum sg e f^T + 1/2a (r0 (F w)^T + (E w) l0v^T)
-      double r0[M], ew[M], fw[M];
-      r0[0] = 1.0;
+      S.factor();
+      // the right-hand sides: w r (LDA part) and w sum K+ U, or their
+      // difference where only the N residual is needed
+      double b[M], x[M], p, Q[D], kun[M], ub[M], pu, Qu[D];
+      if constexpr (NDIS) ku.total(pt, kun);
 #pragma unroll
-      for (int x = 0; x < D; ++x) r0[1 + x] = st.V[x];
-      r0[M - 1] = st.H;
-      double vw = 0.0;
-#pragma unroll
-      for (int x = 0; x < D; ++x) vw += st.V[x] * w[x];
-      ew[0] = 0.0;
-      fw[0] = -vw;
-#pragma unroll
-      for (int x = 0; x < D; ++x) {
-        ew[1 + x] = w[x];
-        fw[1 + x] = w[x];
-      }
-      ew[M - 1] = vw;
-      fw[M - 1] = 0.0;
-      double TV[D], VTV = 0.0;
-#pragma unroll
-      for (int x = 0; x < D; ++x) {
-        double t = 0.0;
-#pragma unroll
-        for (int y = 0; y < D; ++y) t += T[x][y] * st.V[y];
-        TV[x] = t;
-        VTV += st.V[x] * t;
-      }
-      const double c1 = ssg * i2a2;
-      constexpr int R = NDIS ? 2 : 1;
-      double A[M][M];
-      double B[M][R];
-#pragma unroll
-      for (int i = 0; i < M; ++i)
-#pragma unroll
-        for (int j = 0; j < M; ++j) {
-          // 1/2 sum_n sg_n e_n f_n^T
-          double et = 0.0;
-          if (i >= 1 && i <= D) {
-            if (j == 0) et = -TV[i - 1];
-            else if (j <= D) et = T[i - 1][j - 1];
-          } else if (i == M - 1) {
-            if (j == 0) et = -VTV;
-            else if (j <= D) et = TV[j - 1];
-          }
-          A[i][j] = ((i == j) ? sl0 : 0.0) + c1 * r0[i] * l0v[j] + 0.5 * et + i2a * (r0[i] * fw[j] + ew[i] * l0v[j]);
-        }
-#pragma unroll
-      for (int i = 0; i < M; ++i) B[i][0] = r[i];
-      if constexpr (NDIS) {
-#pragma unroll
-        for (int i = 0; i < M; ++i) B[i][1] = 0.0;
-#pragma unroll
-        for (int n = 0; n < ND; ++n) {
-          double un[M], z[M];
-#pragma unroll
-          for (int k = 0; k < M; ++k) un[k] = Uq(n, k);
-          kplus(node_at(n), un, z);
-#pragma unroll
-          for (int k = 0; k < M; ++k) B[k][1] += z[k];
-        }
-      }
-      solve_pp<M, R>(A, B);
-      double x[M];
-#pragma unroll
-      for (int k = 0; k < M; ++k) x[k] = B[k][0] * wj;
+      for (int k = 0; k < M; ++k) b[k] = wj * ((NDIS && !DIS2) ? r[k] - kun[k] : r[k]);
+      S.solve(pt, b, x, p, Q);
+      if constexpr (DIS2) S.solve(pt, kun, ub, pu, Qu);
 #pragma unroll
       for (int n = 0; n < ND; ++n) {
         const NodeK kn = node_at(n);
-        double t[M];
-        kplus(kn, x, t);
-#pragma unroll
-        for (int k = 0; k < M; ++k) lda[n][k] += t[k];
+        if constexpr (DIS2 || !NDIS) pt.apply(kn, x, p, Q, lda[n]);
         if constexpr (NDIS) {
           double du[M];
 #pragma unroll
-          for (int k = 0; k < M; ++k) du[k] = wj * (Uq(n, k) - B[k][R - 1]);
-          kplus(kn, du, t);
-#pragma unroll
-          for (int k = 0; k < M; ++k) dis[n][k] += t[k];
+          for (int k = 0; k < M; ++k) du[k] = DIS2 ? wj * (Uq(n, k) - ub[k]) : wj * Uq(n, k) + x[k];
+          pt.apply(kn, du, DIS2 ? dis[n] : lda[n]);
         }
       }
     }
@@ -843,7 +894,7 @@ __device__ __forceinline__ void cell_residual(const double *__restrict__ tab, co
     const double gm1 = pp.p0 - 1.0;
     const double(&Jq)[D][D] = Jinv[0];
     // LDS column: [q M, q M + M) the divergence of q, then (V, a, H) of q;
-    // [NQ M + 2 M q, + M) x_q, [NQ M + 2 M q + M, + M) w_q ub_q
+    // [NQ M + R M q, + R M) its solutions
     double *const qx = lds_div + static_cast<size_t>(NQ) * M * stride;
 #pragma unroll 1
     for (int q = 0; q < NQ; ++q) {
@@ -865,93 +916,73 @@ __device__ __forceinline__ void cell_residual(const double *__restrict__ tab, co
       }
       const EulerState<double, D> st = euler_state<double, D>(uq, double(pp.p0));
       bad = bad || st.bad;
-      const double i2a = 0.5 * st.inv_a, i2a2 = i2a * st.inv_a;
-      double l0v[M];
-      l0v[0] = 0.5 * gm1 * st.v2;
-#pragma unroll
-      for (int x = 0; x < D; ++x) l0v[1 + x] = -gm1 * st.V[x];
-      l0v[M - 1] = gm1;
-      double sl0 = 0.0, ssg = 0.0, w[D], T[D][D], B[M][2];
-#pragma unroll
-      for (int x = 0; x < D; ++x) {
-        w[x] = 0.0;
-#pragma unroll
-        for (int y = 0; y < D; ++y) T[x][y] = 0.0;
-      }
-#pragma unroll
-      for (int k = 0; k < M; ++k) {
-        B[k][0] = r[k];
-        B[k][1] = 0.0;
-      }
+      const EulerPoint<D> pt = euler_point<D>(st, gm1);
+      EulerSum<D> S;
+      EulerKU<D> ku;
+      S.clear();
+      ku.clear();
 #pragma unroll
       for (int n = 0; n < ND; ++n) {
-        const EulerNodeK<D> k = euler_node_k<D, ND>(Jq, dvk, n, st.V, st.a);
+        const EulerNodeK<D> k = euler_node_k<D, ND>(Jq, dvk, n, pt.V, pt.a);
         lmax = fmax(lmax, k.emax);
-        sl0 += k.l0;
-        ssg += k.sg;
-#pragma unroll
-        for (int x = 0; x < D; ++x) {
-          w[x] += k.dl * k.nh[x];
-#pragma unroll
-          for (int y = 0; y < D; ++y) T[x][y] += k.sg * k.nh[x] * k.nh[y];
-        }
-        double un[M], z[M];
+        S.add(k);
+        double un[M];
 #pragma unroll
         for (int c = 0; c < M; ++c) un[c] = Uq(n, c);
-        euler_kplus<D>(k, l0v, st.V, st.H, st.a, i2a, i2a2, un, z);
-#pragma unroll
-        for (int c = 0; c < M; ++c) B[c][1] += z[c];
+        ku.add(pt, k, un);
       }
-      double A[M][M];
-      euler_kplus_sum<D>(sl0, ssg, w, T, l0v, st.V, st.H, i2a, i2a2, A);
-      solve_pp<M, 2>(A, B);
+      S.factor();
+      double b[M], kun[M], x[M], p, Q[D];
+      ku.total(pt, kun);
 #pragma unroll
-      for (int x = 0; x < D; ++x) lds_div[(q * M + x) * stride] = st.V[x];
-      lds_div[(q * M + D) * stride] = st.a;
-      lds_div[(q * M + D + 1) * stride] = st.H;
+      for (int k = 0; k < M; ++k) b[k] = wj * (DIS2 ? r[k] : r[k] - kun[k]);
+      S.solve(pt, b, x, p, Q);
 #pragma unroll
-      for (int k = 0; k < M; ++k) {
-        qx[(2 * M * q + k) * stride] = B[k][0] * wj;
-        qx[(2 * M * q + M + k) * stride] = B[k][1] * wj;
+      for (int k = 0; k < M; ++k) qx[(R * M * q + k) * stride] = x[k];
+      if constexpr (DIS2) {
+        S.solve(pt, kun, x, p, Q);
+#pragma unroll
+        for (int k = 0; k < M; ++k) qx[(R * M * q + M + k) * stride] = x[k];
       }
+#pragma unroll
+      for (int d = 0; d < D; ++d) lds_div[(q * M + d) * stride] = pt.V[d];
+      lds_div[(q * M + D) * stride] = pt.a;
+      lds_div[(q * M + D + 1) * stride] = pt.H;
     }
 #pragma unroll 1
     for (int q = 0; q < NQ; ++q) {
-      double V[D], x[M], wub[M];
-#pragma unroll
-      for (int d = 0; d < D; ++d) V[d] = lds_div[(q * M + d) * stride];
-      const double a = lds_div[(q * M + D) * stride];
-      const double H = lds_div[(q * M + D + 1) * stride];
-#pragma unroll
-      for (int k = 0; k < M; ++k) {
-        x[k] = qx[(2 * M * q + k) * stride];
-        wub[k] = qx[(2 * M * q + M + k) * stride];
-      }
-      const double wj = tab[O::w + q] * detJ[0];
-      const double ia = recip(a);
-      const double i2a = 0.5 * ia, i2a2 = i2a * ia;
+      EulerPoint<D> pt;
+      double x[M], ub[M], Q[D];
       double v2 = 0.0;
 #pragma unroll
-      for (int d = 0; d < D; ++d) v2 += V[d] * V[d];
-      double l0v[M];
-      l0v[0] = 0.5 * gm1 * v2;
+      for (int d = 0; d < D; ++d) {
+        pt.V[d] = lds_div[(q * M + d) * stride];
+        v2 += pt.V[d] * pt.V[d];
+      }
+      pt.a = lds_div[(q * M + D) * stride];
+      pt.H = lds_div[(q * M + D + 1) * stride];
+      pt.ia = recip(pt.a);
+      pt.hv = 0.5 * v2;
+      pt.ga = gm1 * pt.ia;
 #pragma unroll
-      for (int d = 0; d < D; ++d) l0v[1 + d] = -gm1 * V[d];
-      l0v[M - 1] = gm1;
+      for (int k = 0; k < M; ++k) x[k] = qx[(R * M * q + k) * stride];
+      if constexpr (DIS2) {
+#pragma unroll
+        for (int k = 0; k < M; ++k) ub[k] = qx[(R * M * q + M + k) * stride];
+      }
+#pragma unroll
+      for (int d = 0; d < D; ++d) Q[d] = x[1 + d] - pt.V[d] * x[0];
+      const double p = pt.p_of(x);
+      const double wj = tab[O::w + q] * detJ[0];
       const double *dvk = tab + O::dVT + q * D * ND;
 #pragma unroll
       for (int n = 0; n < ND; ++n) {
-        const EulerNodeK<D> k = euler_node_k<D, ND>(Jq, dvk, n, V, a);
-        double t[M], du[M];
-        euler_kplus<D>(k, l0v, V, H, a, i2a, i2a2, x, t);
+        const EulerNodeK<D> k = euler_node_k<D, ND>(Jq, dvk, n, pt.V, pt.a);
+        double du[M];
 #pragma unroll
-        for (int c = 0; c < M; ++c) {
-          lda[n][c] += t[c];
-          du[c] = wj * Uq(n, c) - wub[c];
-        }
-        euler_kplus<D>(k, l0v, V, H, a, i2a, i2a2, du, t);
-#pragma unroll
-        for (int c = 0; c < M; ++c) dis[n][c] += t[c];
+        for (int c = 0; c < M; ++c) du[c] = DIS2 ? wj * (Uq(n, c) - ub[c]) : wj * Uq(n, c) + x[c];
+        if constexpr (DIS2) pt.apply(k, x, p, Q, lda[n]);
+        pt.apply(k, du, DIS2 ? dis[n] : lda[n]);
       }
     }
   } else {
@@ -981,16 +1012,11 @@ __device__ __forceinline__ void cell_residual(const double *__restrict__ tab, co
   }
 
   // ---- blend / limit -------------------------------------------------------
-  if constexpr (SC == SC_LDA) {
+  if constexpr (SC == SC_LDA || SC == SC_N) {
 #pragma unroll
     for (int n = 0; n < ND; ++n)
 #pragma unroll
       for (int k = 0; k < M; ++k) phi[n][k] = lda[n][k];
-  } else if constexpr (SC == SC_N) {
-#pragma unroll
-    for (int n = 0; n < ND; ++n)
-#pragma unroll
-      for (int k = 0; k < M; ++k) phi[n][k] = lda[n][k] + dis[n][k];
   } else if constexpr (SC == SC_B && (PREC == 2 || PREC == 5)) {
     // external nodal coefficient; below 1e-6 at every node the cell keeps
     // its LDA residuals
@@ -1034,12 +1060,12 @@ __device__ __forceinline__ void cell_residual(const double *__restrict__ tab, co
       double sx = 0.0;
 #pragma unroll
       for (int n = 0; n < ND; ++n) {
-        xs[n] = fmax((lda[n][k] + dis[n][k]) * itot, 0.0) + 1.e-12;
+        xs[n] = fmax((DIS2 ? lda[n][k] + dis[n][k] : lda[n][k]) * itot, 0.0) + 1.e-12;
         sx += xs[n];
       }
 #pragma unroll
       for (int n = 0; n < ND; ++n) {
-        const double psi = lim ? xs[n] / sx * tot : lda[n][k] + dis[n][k];
+        const double psi = lim ? xs[n] / sx * tot : (DIS2 ? lda[n][k] + dis[n][k] : lda[n][k]);
         phi[n][k] = (SC == SC_BPSI) ? (1.0 - theta) * lda[n][k] + theta * psi : psi;
       }
     }

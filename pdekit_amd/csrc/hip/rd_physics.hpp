@@ -37,37 +37,28 @@ struct PhysParams
 };
 
 // 1/x for |x| and 1/|x| in the normal range: the hardware reciprocal
-// estimate (relative error below 2^-22) refined by two Newton steps
-// y <- y + y (1 - x y), each of which squares the relative error, so the
-// result is within an ulp or two of the IEEE quotient at a third of the
+// estimate y (relative error below 2^-22) with the error e = 1 - x y taken out
+// to third order, y (1 + e + e^2): its truncation error e^3 is below 2^-66, so
+// the result is within an ulp or two of the IEEE quotient at a third of the
 // instructions of the IEEE division sequence. x = 0 gives NaN.
 __device__ __forceinline__ double recip(double x)
 {
-  double y = __builtin_amdgcn_rcp(x);
-  double e = fma(-x, y, 1.0);
-  y = fma(y, e, y);
-  e = fma(-x, y, 1.0);
-  return fma(y, e, y);
+  const double y = __builtin_amdgcn_rcp(x);
+  const double e = fma(-x, y, 1.0);
+  return fma(y, fma(e, e, e), y);
 }
 
 // sqrt(x) and 1/sqrt(x) for x > 0 in the normal range, from one hardware
-// reciprocal square root estimate y: Goldschmidt's coupled iteration on
-// g = x y -> sqrt(x) and h = y / 2 -> 1 / (2 sqrt(x)) (r = 1/2 - g h,
-// g <- g + g r, h <- h + h r; two steps take the relative error from 2^-22
-// below 2^-60), then one correction of g from its residual x - g^2. Replaces
-// a square root and a division. x = 0 gives NaN for both.
+// reciprocal square root estimate y with its error e = 1 - x y^2 taken out to
+// third order, y (1 + e/2 + 3 e^2 / 8) (the next term of the series, 5 e^3 /
+// 16, is below 2^-66). Replaces a square root and a division; x = 0 gives NaN
+// for both.
 __device__ __forceinline__ void sqrt_rsqrt(double x, double &s, double &rs)
 {
   const double y = __builtin_amdgcn_rsq(x);
-  double g = x * y, h = 0.5 * y;
-  double r = fma(-g, h, 0.5);
-  g = fma(g, r, g);
-  h = fma(h, r, h);
-  r = fma(-g, h, 0.5);
-  g = fma(g, r, g);
-  h = fma(h, r, h);
-  s = fma(fma(-g, g, x), h, g);
-  rs = 2.0 * h;
+  const double e = fma(-x * y, y, 1.0);
+  rs = fma(y * e, fma(0.375, e, 0.5), y);
+  s = x * rs;
 }
 
 // Thermodynamic state at a point (Euler); inv_a = 1 / a.
