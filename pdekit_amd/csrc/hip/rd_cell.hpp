@@ -569,11 +569,72 @@ __device__ __forceinline__ void cell_residual(const double *__restrict__ tab, co
   }
 
   // ---- P+1 flux element: divergence of the interpolated flux at q ---------
+  {
+  double divr[NQ][M];
+  // P1 simplices of the Euler equations: their P2 flux element has the
+  // vertices and the edge midpoints as nodes, so with b_i the gradients of the
+  // vertex functions l_i,
+  //   div F = sum_i l_i E_i,  E_i = 4 (F_i . b_i + sum_{j != i} F_ij . b_j) - sum_k F_k . b_k;
+  // the state at a vertex is the vertex's, at a midpoint half the sum of two,
+  // and F(x / 2) = F(x) / 2. 10 (3D) or 6 (2D) point fluxes are contracted
+  // with 16 (9) vectors and D + 1 vectors E_i interpolated, where the general
+  // form below takes the fluxes of every node to every quadrature point: 470
+  // instead of 1 700 instructions of a P1 tetrahedron's 5 500 (PSI / LDA
+  // blend, 5.3 M cells: with the cap of PatchMinWaves 1.44 -> 1.15 ms).
+  constexpr bool P1S = (M > 1) && AFFINE && (ND == D + 1);
+  if constexpr (P1S) {
+    double b[ND][D], A[ND][M], C[M];
+#pragma unroll
+    for (int n = 0; n < ND; ++n) {
+#pragma unroll
+      for (int x = 0; x < D; ++x) {
+        double t = 0.0;
+#pragma unroll
+        for (int xi = 0; xi < D; ++xi) t += Jinv[0][x][xi] * tab[O::dVT + xi * ND + n];
+        b[n][x] = t;
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < M; ++k) C[k] = 0.0;
+#pragma unroll
+    for (int i = 0; i < ND; ++i) {
+      const EulerState<double, D> st = euler_state<double, D>(U[i], double(pp.p0));
+      bad = bad || st.bad;
+      double c[M];
+#pragma unroll
+      for (int k = 0; k < M; ++k) c[k] = 0.0;
+      euler_flux_add<D>(U[i], st, b[i], c);
+#pragma unroll
+      for (int k = 0; k < M; ++k) {
+        C[k] += c[k];
+        A[i][k] = 2.0 * c[k];
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < ND; ++i)
+#pragma unroll
+      for (int j = i + 1; j < ND; ++j) {
+        double s[M];
+#pragma unroll
+        for (int k = 0; k < M; ++k) s[k] = U[i][k] + U[j][k];
+        const EulerState<double, D> st = euler_state<double, D>(s, double(pp.p0));
+        bad = bad || st.bad;
+        euler_flux_add<D>(s, st, b[j], A[i]);
+        euler_flux_add<D>(s, st, b[i], A[j]);
+      }
+#pragma unroll
+    for (int q = 0; q < NQ; ++q)
+#pragma unroll
+      for (int k = 0; k < M; ++k) {
+        double t = 0.0;
+#pragma unroll
+        for (int n = 0; n < ND; ++n) t += tab[O::V + q * ND + n] * A[n][k];
+        divr[q][k] = 2.0 * t - C[k];
+      }
+  } else {
   // The flux-node loop stays rolled: each trip reads one row of Vsf and one
   // [D][NQ] slab of dVf with scalar loads, so the table never has to be held
   // in (and spilled from) scalar registers as a whole.
-  {
-  double divr[NQ][M];
 #pragma unroll
   for (int q = 0; q < NQ; ++q)
 #pragma unroll
@@ -594,6 +655,21 @@ __device__ __forceinline__ void cell_residual(const double *__restrict__ tab, co
       s[k] = t;
     }
     double F[D][M];
+    double G[AFFINE ? D : 1][M];
+    if constexpr (M > 1 && AFFINE) {
+      // the contravariant fluxes straight from the state
+      const EulerState<double, D> st = euler_state<double, D>(s, double(pp.p0));
+      bad = bad || st.bad;
+#pragma unroll
+      for (int xi = 0; xi < D; ++xi) {
+        double b[D];
+#pragma unroll
+        for (int d = 0; d < D; ++d) b[d] = Jinv[0][d][xi];
+#pragma unroll
+        for (int k = 0; k < M; ++k) G[xi][k] = 0.0;
+        euler_flux_add<D>(s, st, b, G[xi]);
+      }
+    } else {
     PhysParams ppf = pp;
     if constexpr (PH == PH_ROTATION2D) {
       // the velocity (y, -x) at the flux node's coordinates Vgf X
@@ -606,7 +682,6 @@ __device__ __forceinline__ void cell_residual(const double *__restrict__ tab, co
       ppf.p1 = -xf[0];
     }
     point_flux<PH, double>(s, ppf, F, bad);
-    double G[AFFINE ? D : 1][M];
     if constexpr (AFFINE) {
 #pragma unroll
       for (int xi = 0; xi < D; ++xi)
@@ -617,6 +692,7 @@ __device__ __forceinline__ void cell_residual(const double *__restrict__ tab, co
           for (int d = 0; d < D; ++d) t += Jinv[0][d][xi] * F[d][k];
           G[xi][k] = t;
         }
+    }
     }
 #pragma unroll
     for (int q = 0; q < NQ; ++q) {
@@ -646,6 +722,7 @@ __device__ __forceinline__ void cell_residual(const double *__restrict__ tab, co
         }
       }
     }
+  }
   }
   if constexpr (PREC == 3 || PREC == 5) {
 #pragma unroll
@@ -706,9 +783,7 @@ __device__ __forceinline__ void cell_residual(const double *__restrict__ tab, co
   // P1 simplices of the Euler physics (affine, D + 1 nodes): the basis
   // gradients, and with them the geometric part of every node's K+
   // parameters, are the same at every quadrature point; formed once per cell
-  // (not for the P1 tetrahedra's LDA, which the compiler fits in 2 waves
-  // without the registers they take)
-  constexpr bool CG = (M > 1) && AFFINE && (ND == D + 1) && !(D == 3 && SC == SC_LDA);
+  constexpr bool CG = (M > 1) && AFFINE && (ND == D + 1);
   EulerNodeG<D> cg[CG ? ND : 1];
   if constexpr (CG) {
 #pragma unroll
@@ -830,8 +905,8 @@ __device__ __forceinline__ void cell_residual(const double *__restrict__ tab, co
         else
           return euler_node_k<D, ND>(Jq, dvk, n, pt.V, pt.a);
       };
-      // 3D: recompute in the application instead of keeping ND sets
-      constexpr bool KEEP = (D == 2);
+      // 3D P2: recompute in the application instead of keeping ND sets
+      constexpr bool KEEP = (D == 2) || CG;
       NodeK nk[KEEP ? ND : 1];
       EulerSum<D> S;
       S.clear();
@@ -856,10 +931,9 @@ __device__ __forceinline__ void cell_residual(const double *__restrict__ tab, co
         } else if constexpr (SC == SC_LDA) {
           // an opaque copy of the index: the parameters are recomputed here,
           // not kept alive from the loop over S (which common-subexpression
-          // elimination would otherwise do); measured faster for LDA (fewer
-          // registers: 2 waves per SIMD on P1, no scratch on P2) and slower
-          // for the dissipative schemes, whose second application per node
-          // reuses the parameters
+          // elimination would otherwise do); measured faster for LDA (no
+          // scratch) and slower for the dissipative schemes, whose second
+          // application per node reuses the parameters
           int nn = n;
           asm volatile("" : "+s"(nn));
           return node_k(nn);
@@ -1222,11 +1296,12 @@ struct PatchSize
 
 // Waves per SIMD the register allocation of a patch kernel must leave room
 // for: 5 for the scalar affine P1 / P2 cells (at most 96 VGPRs, measured
-// faster than 4 waves); 2 for the 2D Euler cells of up to 4 nodes (little or
-// no scratch, measured faster than 1 wave); the others keep the compiler's
-// choice (the FP64 3D Euler cells run as fast at 1 wave, where capping them
-// at 2 spills a few hundred bytes per thread to scratch memory; the 2D Euler
-// P2 / Q2 / P3 cells spill 250-1600 bytes per thread at 2 waves). The linear
+// faster than 4 waves); 2 for the Euler cells of up to 4 nodes, which need at
+// most 256 registers but for the tetrahedra's blends (152 bytes of scratch per
+// lane): 1.57 M P1 tetrahedra per sweep at 1 and 2 waves: N 289 -> 223 us, PSI
+// / LDA blend 412 -> 336 us (the second wave covers the first's waits, a third
+// of its life). The others keep the compiler's choice: the P2 / Q2 / P3 Euler
+// cells fill the LDS at 1 wave, so that the cap only adds scratch. The linear
 // sweeps (PREC 4, J delta per cell) are bound by the Jacobians' bandwidth and
 // keep 4 waves (2 for blocks of more than 24 unknowns).
 template <int M, int ND, bool AFFINE, int SC, int PREC>
@@ -1234,7 +1309,7 @@ struct PatchMinWaves
 {
   static constexpr int value =
       (PREC == 4) ? (ND * M <= 24 ? 4 : 2)
-                  : ((M == 1 && ND <= 6 && AFFINE) ? 5 : ((M == 4 && ND <= 4) ? 2 : 1));
+                  : ((M == 1 && ND <= 6 && AFFINE) ? 5 : ((M > 1 && ND <= 4) ? 2 : 1));
 };
 
 // Dynamic LDS of one patch workgroup of P cells, in doubles: node state
@@ -1424,12 +1499,7 @@ __device__ __forceinline__ void patch_body(const PatchArgs &a, uint32_t pl, doub
   // work: at the finish, those loads behind the node id were two rounds of
   // memory latency per node that no other wave hid (a sixth of the wave's
   // life on the P2 triangles).
-  // (the Euler cells only, not the P1 tetrahedra's LDA, which the compiler
-  // fits in 2 waves)
-  constexpr int FP = (M > 1 && PatchMinWaves<M, ND, AFFINE, SC, PREC>::value == 1 && PREC != 4 &&
-                      (ND > 4 || SC != SC_LDA))
-                         ? 4
-                         : 0;
+  constexpr int FP = (M > 1 && PatchMinWaves<M, ND, AFFINE, SC, PREC>::value == 1 && PREC != 4) ? 4 : 0;
   constexpr int FPS = FP > 0 ? FP : 1;
   uint32_t pg[FPS], psp[FPS];
   double pv[FPS];

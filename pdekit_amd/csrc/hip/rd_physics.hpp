@@ -92,6 +92,25 @@ __device__ __forceinline__ EulerState<T, D> euler_state(const T *s, T gamma)
   return st;
 }
 
+// out += F(s) . b for the Euler fluxes at a state of momentum s[1..D] and a
+// direction b (Euler fluxes contracted before they are formed: 3 D + 1
+// operations instead of D (D + 1) for the fluxes and D (D + 2) for the product).
+template <int D>
+__device__ __forceinline__ void euler_flux_add(const double *s, const EulerState<double, D> &st, const double *b,
+                                               double *out)
+{
+  double mb = 0.0;
+#pragma unroll
+  for (int d = 0; d < D; ++d) mb += s[1 + d] * b[d];
+  out[0] += mb;
+#pragma unroll
+  for (int d = 0; d < D; ++d) {
+    const double t = out[1 + d] + st.V[d] * mb;
+    out[1 + d] = t + st.P * b[d];
+  }
+  out[D + 1] += st.H * mb;
+}
+
 // Physical flux F[d][k] at a state.
 template <int PH, typename T>
 __device__ __forceinline__ void point_flux(const T *s, const PhysParams &pp, T F[][PhysTraits<PH>::M], bool &bad)
