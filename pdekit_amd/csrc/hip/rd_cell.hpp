@@ -521,6 +521,59 @@ struct EulerKU
   }
 };
 
+// Waves per SIMD the register allocation of a patch kernel must leave room
+// for: 5 for the scalar affine P1 / P2 cells (at most 96 VGPRs, measured
+// faster than 4 waves); 2 for the Euler cells of up to 4 nodes, which need at
+// most 256 registers but for the tetrahedra's blends (152 bytes of scratch per
+// lane): 1.57 M P1 tetrahedra per sweep at 1 and 2 waves: N 289 -> 223 us, PSI
+// / LDA blend 412 -> 336 us (the second wave covers the first's waits, a third
+// of its life); 2 for the schemes with one residual sum per node (LDA, N, PSI)
+// on P2 triangles and for the LDA of P2 tetrahedra with the 4-point rule, which
+// need 256 registers or a few more, their pair sums in phases (PatchWork) so
+// that 8 waves fit the LDS too: 131 072 P2 triangles LDA 42.0 -> 33.9 us, N 45.5
+// -> 38.6 us, 0.20 M P2 tetrahedra LDA 146 -> 125 us a sweep. The others keep
+// the compiler's choice, 1 wave: at 2 the B scheme of P2 triangles takes 220
+// bytes of scratch (54 -> 60 us), Q2 quadrilaterals 312 (65 536 cells LDA 44 ->
+// 55 us), the P2 tetrahedra's N 172 (137 -> 151 us). The linear sweeps (PREC 4,
+// J delta per cell) are bound by the Jacobians' bandwidth and keep 4 waves (2
+// for blocks of more than 24 unknowns).
+template <int M, int ND, int NQ, bool AFFINE, int SC, int PREC>
+struct PatchMinWaves
+{
+  static constexpr bool one_sum = SC == SC_LDA || SC == SC_N || SC == SC_PSI;
+  static constexpr bool two_p2 =
+      AFFINE && ((M == 4 && ND == 6 && one_sum) || (M == 5 && ND == 10 && NQ == 4 && SC == SC_LDA));
+  static constexpr int value = (PREC == 4)                        ? (ND * M <= 24 ? 4 : 2)
+                               : (M == 1 && ND <= 6 && AFFINE)    ? 5
+                               : (M > 1 && (ND <= 4 || two_p2)) ? 2
+                                                                  : 1;
+};
+
+// Use of a patch workgroup's LDS work region, in doubles per cell. `column`:
+// what the cell computation keeps in its own column, the flux divergence at
+// the quadrature points or, with `two` passes over them (the dissipative
+// schemes of the 3D P2 cells, see cell_residual), also the `rhs` solutions of
+// every point. Afterwards the region carries the (cell, node) pair sums, `comps`
+// of the M + 1 components at a time: all of them at once, or as many as the
+// column holds where the region would otherwise grow for the pairs and the LDS,
+// not the registers, would then limit the waves: the kernels of 2 waves on more
+// than 4 nodes, and the two-pass ones (0.20 M P2 tetrahedra N 143 -> 137 us). On
+// the others the phases' barriers cost more than they give (P2 triangles at 1
+// wave 42 -> 46 us, Q2 44 -> 48 us).
+template <int D, int ND, int NQ, bool AFFINE, int M, int SC, int PREC>
+struct PatchWork
+{
+  static constexpr int rhs = (SC == SC_B || SC == SC_BPSI) ? 2 : 1;
+  static constexpr bool two =
+      D == 3 && SC != SC_LDA && AFFINE && M == D + 2 && PREC != 4 && NQ * (1 + rhs) * M <= ND * (M + 1);
+  static constexpr int column = (PREC == 4) ? 0 : (two ? NQ * (1 + rhs) * M : NQ * M);
+  static constexpr bool phased = M > 1 && PREC != 4 && ND > 4 && ND * (M + 1) > column &&
+                                 (two || PatchMinWaves<M, ND, NQ, AFFINE, SC, PREC>::value == 2);
+  static constexpr int comps = phased ? (column >= ND ? column / ND : 1) : M + 1;
+  static constexpr int per_cell =
+      column > comps * ND ? (column > M + 1 ? column : M + 1) : (comps * ND > M + 1 ? comps * ND : M + 1);
+};
+
 // Residuals phi[ND][M] and wave speed of one element from its vertex
 // coordinates X and nodal state U. lds_div: this thread's slice of NQ*M
 // doubles of LDS (stride `stride` between entries) that carries the flux
@@ -767,8 +820,8 @@ __device__ __forceinline__ void cell_residual(const double *__restrict__ tab, co
   for (int k = 0; k < M; ++k) fint[k] = 0.0;
   double vol = 0.0;
 
-  // TWO: the dissipative schemes of the 3D P2 cells (affine, NQ (1 + R) M <=
-  // ND (M + 1), R right-hand sides) in two passes over the quadrature points,
+  // TWO: the dissipative schemes of the 3D P2 cells (affine, R right-hand
+  // sides) in two passes over the quadrature points,
   // so that neither holds the K+ parameters of all nodes beside the residual
   // sums:
   //   1. per point q: S_q = sum_n K+_n (one evaluation of each node's
@@ -778,7 +831,7 @@ __device__ __forceinline__ void cell_residual(const double *__restrict__ tab, co
   //   2. per point q again, every node: its K+ products added to its sums (a
   //      second evaluation of the parameters).
   constexpr int R = DIS2 ? 2 : 1;
-  constexpr bool TWO = (D == 3) && NDIS && AFFINE && DLDS && (M == D + 2) && (NQ * (1 + R) * M <= ND * (M + 1));
+  constexpr bool TWO = DLDS && PatchWork<D, ND, NQ, AFFINE, M, SC, PREC>::two;
 
   // P1 simplices of the Euler physics (affine, D + 1 nodes): the basis
   // gradients, and with them the geometric part of every node's K+
@@ -1294,68 +1347,22 @@ struct PatchSize
   static constexpr int value = (M == 1 && ND <= 6) ? 256 : ((M == 5 && ND > 4) ? 64 : 128);
 };
 
-// Waves per SIMD the register allocation of a patch kernel must leave room
-// for: 5 for the scalar affine P1 / P2 cells (at most 96 VGPRs, measured
-// faster than 4 waves); 2 for the Euler cells of up to 4 nodes, which need at
-// most 256 registers but for the tetrahedra's blends (152 bytes of scratch per
-// lane): 1.57 M P1 tetrahedra per sweep at 1 and 2 waves: N 289 -> 223 us, PSI
-// / LDA blend 412 -> 336 us (the second wave covers the first's waits, a third
-// of its life). The others keep the compiler's choice: the P2 / Q2 / P3 Euler
-// cells fill the LDS at 1 wave, so that the cap only adds scratch. The linear
-// sweeps (PREC 4, J delta per cell) are bound by the Jacobians' bandwidth and
-// keep 4 waves (2 for blocks of more than 24 unknowns).
-template <int M, int ND, bool AFFINE, int SC, int PREC>
-struct PatchMinWaves
-{
-  static constexpr int value =
-      (PREC == 4) ? (ND * M <= 24 ? 4 : 2)
-                  : ((M == 1 && ND <= 6 && AFFINE) ? 5 : ((M > 1 && ND <= 4) ? 2 : 1));
-};
-
 // Dynamic LDS of one patch workgroup of P cells, in doubles: node state
-// [maxl][M], the pair offsets of the nodes [maxl] (u16), then a work region
-// shared in turn by the flux-divergence slices, the (cell, node) pair sums
-// and the norm reduction.
-template <int NQ, int ND, int M>
-__host__ __device__ constexpr size_t patch_work_doubles(int P)
-{
-  const size_t div = static_cast<size_t>(NQ) * M * P;
-  const size_t pairs = static_cast<size_t>(P) * ND * (M + 1);
-  const size_t red = static_cast<size_t>(P) * (M + 1);
-  const size_t w = div > pairs ? div : pairs;
-  return w > red ? w : red;
-}
-
+// [maxl][M], the pair offsets of the nodes [maxl] (u16), then a work region of
+// PatchWork::per_cell doubles a cell, shared in turn by the cells' columns, the
+// (cell, node) pair sums and the norm reduction. With a nodal input (PREC 2)
+// its values follow the work region, one per local node; with a source field
+// (PREC 3), M per local node, and with both (PREC 5) M + 1. In a linear sweep
+// (PREC 4) the state differences delta of the patch's nodes follow, [maxl][M]
+// floats.
 __host__ __device__ constexpr size_t patch_coff_doubles(int maxl) { return (static_cast<size_t>(maxl) + 3) / 4; }
 
-template <int NQ, int ND, int M>
+template <class PW, int M, int PREC>
 __host__ __device__ constexpr size_t patch_lds_doubles(int maxl, int P)
 {
-  return static_cast<size_t>(maxl) * M + patch_coff_doubles(maxl) + patch_work_doubles<NQ, ND, M>(P);
-}
-
-// With a nodal input (PREC 2) its values follow the work region, one per
-// local node; with a source field (PREC 3), M per local node. A linear sweep
-// (PREC 4) has no divergence slices: its work region holds the pair sums
-// and the norm reduction, followed by the state differences delta of the
-// patch's nodes, [maxl][M] floats.
-template <int NQ, int ND, int M>
-__host__ __device__ constexpr size_t patch_lin_work_doubles(int P)
-{
-  const size_t pairs = static_cast<size_t>(P) * ND * (M + 1);
-  const size_t red = static_cast<size_t>(P) * (M + 1);
-  return pairs > red ? pairs : red;
-}
-
-template <int NQ, int ND, int M, int PREC>
-__host__ __device__ constexpr size_t patch_lds_doubles_prec(int maxl, int P)
-{
-  if (PREC == 4)
-    return static_cast<size_t>(maxl) * M + patch_coff_doubles(maxl) + patch_lin_work_doubles<NQ, ND, M>(P) +
-           (static_cast<size_t>(maxl) * M + 1) / 2;
-  return patch_lds_doubles<NQ, ND, M>(maxl, P) +
-         (PREC == 2 ? static_cast<size_t>(maxl)
-                    : (PREC == 3 ? static_cast<size_t>(maxl) * M : (PREC == 5 ? static_cast<size_t>(maxl) * (M + 1) : 0)));
+  const size_t n = static_cast<size_t>(maxl);
+  return n * M + patch_coff_doubles(maxl) + static_cast<size_t>(P) * PW::per_cell +
+         (PREC == 2 ? n : (PREC == 3 ? n * M : (PREC == 4 ? (n * M + 1) / 2 : (PREC == 5 ? n * (M + 1) : 0))));
 }
 
 // Finishes node g from its sums acc[M + 1] (residual sum, wave-speed sum);
@@ -1489,8 +1496,9 @@ __device__ __forceinline__ void patch_body(const PatchArgs &a, uint32_t pl, doub
 #pragma unroll
     for (int n = 0; n < ND; ++n) lc[n] = a.lconn[static_cast<size_t>(n) * a.ne + e];
   }
-  double *nodal_l = work + patch_work_doubles<NQ, ND, M>(PATCH);  // PREC 2 and 3 only
-  float *delta_l = reinterpret_cast<float *>(work + patch_lin_work_doubles<NQ, ND, M>(PATCH));  // PREC 4 only
+  using PW = PatchWork<D, ND, NQ, AFFINE, M, SC, PREC>;
+  double *nodal_l = work + static_cast<size_t>(PATCH) * PW::per_cell;  // PREC 2, 3 and 5 only
+  float *delta_l = reinterpret_cast<float *>(nodal_l);                 // PREC 4 only
   // (no global store before the cell work: the table loads stay scalar)
   const int ninner = static_cast<int>(a.pn_inner[p]);
   // The kernels at 1 wave per SIMD load what the node finish needs of the
@@ -1499,7 +1507,7 @@ __device__ __forceinline__ void patch_body(const PatchArgs &a, uint32_t pl, doub
   // work: at the finish, those loads behind the node id were two rounds of
   // memory latency per node that no other wave hid (a sixth of the wave's
   // life on the P2 triangles).
-  constexpr int FP = (M > 1 && PatchMinWaves<M, ND, AFFINE, SC, PREC>::value == 1 && PREC != 4) ? 4 : 0;
+  constexpr int FP = (M > 1 && PatchMinWaves<M, ND, NQ, AFFINE, SC, PREC>::value == 1 && PREC != 4) ? 4 : 0;
   constexpr int FPS = FP > 0 ? FP : 1;
   uint32_t pg[FPS], psp[FPS];
   double pv[FPS];
@@ -1621,34 +1629,36 @@ __device__ __forceinline__ void patch_body(const PatchArgs &a, uint32_t pl, doub
       cell_residual<D, NG, ND, NF, NQ, AFFINE, PH, SC, PREC, true>(a.tab, X, U, ULds<ND, M>{ul, row}, a.pp, phi, wave, bad,
                                                        work + tid, PATCH);
   }
-  __syncthreads();  // the work region changes from divergence slices to pair sums
-  if (active && PREC != 4) {
-#pragma unroll
-    for (int n = 0; n < ND; ++n) {
-      const int slot = coff[lc[n] & LC_MASK] + (lc[n] >> LC_BITS);
-#pragma unroll
-      for (int k = 0; k < M; ++k) work[k * NPAIR + slot] = phi[n][k];
-      work[M * NPAIR + slot] = wave;
-    }
-  }
-  __syncthreads();
-
   const int npair = ecount * ND;
   double sq[M + 1];
 #pragma unroll
   for (int k = 0; k <= M; ++k) sq[k] = 0.0;
-  // node l of the patch; pre: its node id, slot, volume and Dirichlet index
-  // were loaded ahead (pgv, pspv, pvv, pdiv)
-  auto finish_l = [&](const int l, const bool pre, const uint32_t pgv, const uint32_t pspv, const double pvv,
-                      const int pdiv) {
+  // components [c0, c0 + n) of the cell's residuals and wave speed to its pairs
+  auto put_pairs = [&](const int c0, const int n) {
+#pragma unroll
+    for (int i = 0; i < ND; ++i) {
+      const int slot = coff[lc[i] & LC_MASK] + (lc[i] >> LC_BITS);
+#pragma unroll
+      for (int k = 0; k <= M; ++k)
+        if (k >= c0 && k < c0 + n) work[(k - c0) * NPAIR + slot] = (k < M) ? phi[i][k < M ? k : 0] : wave;
+    }
+  };
+  // their sums over the pairs of node l
+  auto sum_pairs = [&](const int l, const int c0, const int n, double (&acc)[M + 1]) {
     const int b = coff[l];
     const int e = (l + 1 < nl) ? static_cast<int>(coff[l + 1]) : npair;
-    double acc[M + 1];
 #pragma unroll
-    for (int k = 0; k <= M; ++k) acc[k] = 0.0;
+    for (int k = 0; k <= M; ++k)
+      if (k >= c0 && k < c0 + n) acc[k] = 0.0;
     for (int i = b; i < e; ++i)
 #pragma unroll
-      for (int k = 0; k <= M; ++k) acc[k] += work[k * NPAIR + i];
+      for (int k = 0; k <= M; ++k)
+        if (k >= c0 && k < c0 + n) acc[k] += work[(k - c0) * NPAIR + i];
+  };
+  // node l of the patch from its sums; pre: its node id, slot, volume and
+  // Dirichlet index were loaded ahead (pgv, pspv, pvv, pdiv)
+  auto finish_l = [&](const int l, const double (&acc)[M + 1], const bool pre, const uint32_t pgv, const uint32_t pspv,
+                      const double pvv, const int pdiv) {
     if (l < ninner) {
       const uint32_t g = pre ? pgv : a.pnodes[s0 + l];
       finish_node<M>(a, g, acc, ul + l * M, pre ? pvv : a.vol[g], pre ? pdiv : a.dir_index[g], sq);
@@ -1671,19 +1681,53 @@ __device__ __forceinline__ void patch_body(const PatchArgs &a, uint32_t pl, doub
       }
     }
   };
-  if constexpr (FP > 0) {
+  if constexpr (PW::phased) {
+    // a few components at a time, the sums of a thread's NPT nodes in
+    // registers; patches of more nodes take another round of all phases
+    constexpr int NPT = 4;
+    for (int l0 = 0; l0 < nl; l0 += NPT * PATCH) {
+      double acc[NPT][M + 1];
 #pragma unroll
-    for (int j = 0; j < FP; ++j) {
-      const int l = tid + j * PATCH;
-      if (l < nl) finish_l(l, true, pg[j], psp[j], pv[j], pdi[j]);
+      for (int c0 = 0; c0 <= M; c0 += PW::comps) {
+        __syncthreads();
+        if (active) put_pairs(c0, PW::comps);
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < NPT; ++j) {
+          const int l = l0 + tid + j * PATCH;
+          if (l < nl) sum_pairs(l, c0, PW::comps, acc[j]);
+        }
+      }
+#pragma unroll
+      for (int j = 0; j < NPT; ++j) {
+        const int l = l0 + tid + j * PATCH;
+        if (l < nl) {
+          if (FP == NPT && l0 == 0)
+            finish_l(l, acc[j], true, pg[j % FPS], psp[j % FPS], pv[j % FPS], pdi[j % FPS]);
+          else
+            finish_l(l, acc[j], false, 0u, 0u, 0.0, 0);
+        }
+      }
     }
-    for (int l = tid + FP * PATCH; l < nl; l += PATCH) finish_l(l, false, 0u, 0u, 0.0, 0);
   } else {
-    (void)pg;
-    (void)psp;
-    (void)pv;
-    (void)pdi;
-    for (int l = tid; l < nl; l += PATCH) finish_l(l, false, 0u, 0u, 0.0, 0);
+    __syncthreads();  // the work region changes from the cells' columns to pair sums
+    if (active && PREC != 4) put_pairs(0, M + 1);
+    __syncthreads();
+    double acc[M + 1];
+    if constexpr (FP > 0) {
+#pragma unroll
+      for (int j = 0; j < FP; ++j) {
+        const int l = tid + j * PATCH;
+        if (l < nl) {
+          sum_pairs(l, 0, M + 1, acc);
+          finish_l(l, acc, true, pg[j], psp[j], pv[j], pdi[j]);
+        }
+      }
+    }
+    for (int l = tid + FP * PATCH; l < nl; l += PATCH) {
+      sum_pairs(l, 0, M + 1, acc);
+      finish_l(l, acc, false, 0u, 0u, 0.0, 0);
+    }
   }
   if (bad) atomicOr(a.status, 1);
   if (a.update && a.outputs) block_sum_store<M>(sq, work, a.norm_partial + static_cast<size_t>(p) * (M + 1));
@@ -1691,7 +1735,7 @@ __device__ __forceinline__ void patch_body(const PatchArgs &a, uint32_t pl, doub
 
 template <int D, int NG, int ND, int NF, int NQ, bool AFFINE, int PH, int SC, int PREC>
 __global__ __launch_bounds__((PatchSize<PhysTraits<PH>::M, ND>::value),
-                             (PatchMinWaves<PhysTraits<PH>::M, ND, AFFINE, SC, PREC>::value)) void rd_patch_kernel(PatchArgs a)
+                             (PatchMinWaves<PhysTraits<PH>::M, ND, NQ, AFFINE, SC, PREC>::value)) void rd_patch_kernel(PatchArgs a)
 {
   extern __shared__ double lds[];
   const uint32_t pl = xcd_block_index();
@@ -1705,7 +1749,7 @@ __global__ __launch_bounds__((PatchSize<PhysTraits<PH>::M, ND>::value),
 // the entries'.
 template <int D, int NG, int ND, int NF, int NQ, bool AFFINE, int PH, int SC, int PREC>
 __global__ __launch_bounds__((PatchSize<PhysTraits<PH>::M, ND>::value),
-                             (PatchMinWaves<PhysTraits<PH>::M, ND, AFFINE, SC, PREC>::value)) void
+                             (PatchMinWaves<PhysTraits<PH>::M, ND, NQ, AFFINE, SC, PREC>::value)) void
 rd_patch_batch_kernel(const PatchArgs *__restrict__ args, const uint32_t *__restrict__ first, int count)
 {
   extern __shared__ double lds[];
