@@ -549,6 +549,15 @@ struct PatchMinWaves
                                                                   : 1;
 };
 
+// Doubles of LDS that carry a cell's flux divergence from the flux nodes to the
+// quadrature points (none where the scheme's own parameters give it).
+template <int D, int ND, int NQ, bool AFFINE, int PH>
+struct CellColumn
+{
+  static constexpr bool linear_flux = ScalarFlux<PH, AFFINE ? D + 1 : (1 << D), ND>::exact;
+  static constexpr int value = linear_flux ? 0 : NQ * PhysTraits<PH>::M;
+};
+
 // Use of a patch workgroup's LDS work region, in doubles per cell. `column`:
 // what the cell computation keeps in its own column, the flux divergence at
 // the quadrature points or, with `two` passes over them (the dissipative
@@ -560,13 +569,14 @@ struct PatchMinWaves
 // than 4 nodes, and the two-pass ones (0.20 M P2 tetrahedra N 143 -> 137 us). On
 // the others the phases' barriers cost more than they give (P2 triangles at 1
 // wave 42 -> 46 us, Q2 44 -> 48 us).
-template <int D, int ND, int NQ, bool AFFINE, int M, int SC, int PREC>
+template <int D, int ND, int NQ, bool AFFINE, int PH, int SC, int PREC>
 struct PatchWork
 {
+  static constexpr int M = PhysTraits<PH>::M;
   static constexpr int rhs = (SC == SC_B || SC == SC_BPSI) ? 2 : 1;
   static constexpr bool two =
       D == 3 && SC != SC_LDA && AFFINE && M == D + 2 && PREC != 4 && NQ * (1 + rhs) * M <= ND * (M + 1);
-  static constexpr int column = (PREC == 4) ? 0 : (two ? NQ * (1 + rhs) * M : NQ * M);
+  static constexpr int column = (PREC == 4) ? 0 : (two ? NQ * (1 + rhs) * M : CellColumn<D, ND, NQ, AFFINE, PH>::value);
   static constexpr bool phased = M > 1 && PREC != 4 && ND > 4 && ND * (M + 1) > column &&
                                  (two || PatchMinWaves<M, ND, NQ, AFFINE, SC, PREC>::value == 2);
   static constexpr int comps = phased ? (column >= ND ? column / ND : 1) : M + 1;
@@ -575,7 +585,7 @@ struct PatchWork
 };
 
 // Residuals phi[ND][M] and wave speed of one element from its vertex
-// coordinates X and nodal state U. lds_div: this thread's slice of NQ*M
+// coordinates X and nodal state U. lds_div: this thread's slice of CellColumn
 // doubles of LDS (stride `stride` between entries) that carries the flux
 // divergence from the flux-node loop to the quadrature loop.
 //
@@ -622,7 +632,14 @@ __device__ __forceinline__ void cell_residual(const double *__restrict__ tab, co
   }
 
   // ---- P+1 flux element: divergence of the interpolated flux at q ---------
-  {
+  // Scalar fluxes that the P+1 element interpolates exactly need none: linear
+  // advection (a u and, rotating, a(x) u with a linear and divergence-free are
+  // of order P + 1) and the Burgers flux (u^2 / 2, u) of first-order elements;
+  // div F at q is then a . grad u = sum_n k_n U_n, from the upwind parameters
+  // that the scheme forms anyway. The loop below would take two thirds of a P3
+  // cell's instructions (101 250 cells N 26.3 -> 20.9 us a sweep without it).
+  constexpr bool LINF = CellColumn<D, ND, NQ, AFFINE, PH>::linear_flux;
+  if constexpr (!LINF) {
   double divr[NQ][M];
   // P1 simplices of the Euler equations: their P2 flux element has the
   // vertices and the edge midpoints as nodes, so with b_i the gradients of the
@@ -831,7 +848,7 @@ __device__ __forceinline__ void cell_residual(const double *__restrict__ tab, co
   //   2. per point q again, every node: its K+ products added to its sums (a
   //      second evaluation of the parameters).
   constexpr int R = DIS2 ? 2 : 1;
-  constexpr bool TWO = DLDS && PatchWork<D, ND, NQ, AFFINE, M, SC, PREC>::two;
+  constexpr bool TWO = DLDS && PatchWork<D, ND, NQ, AFFINE, PH, SC, PREC>::two;
 
   // P1 simplices of the Euler physics (affine, D + 1 nodes): the basis
   // gradients, and with them the geometric part of every node's K+
@@ -843,11 +860,13 @@ __device__ __forceinline__ void cell_residual(const double *__restrict__ tab, co
     for (int n = 0; n < ND; ++n) cg[n] = euler_node_g<D, ND>(Jinv[0], tab + O::dVT, n);
   }
 
-  auto quad_point = [&](const int q, const double (&r)[M], const double (&Jq)[D][D], const double detq) {
+  auto quad_point = [&](const int q, double (&r)[M], const double (&Jq)[D][D], const double detq) {
     const double wj = tab[O::w + q] * detq;
     vol += wj;
+    if constexpr (!LINF) {
 #pragma unroll
-    for (int k = 0; k < M; ++k) fint[k] += wj * r[k];
+      for (int k = 0; k < M; ++k) fint[k] += wj * r[k];
+    }
     const double *dvq = tab + O::dVT + q * D * ND;  // reference gradients [D][ND] at q
 
     if constexpr (PREC == 2 && SC == SC_LDA) {
@@ -915,7 +934,7 @@ __device__ __forceinline__ void cell_residual(const double *__restrict__ tab, co
 #pragma unroll
       for (int xi = 0; xi < D; ++xi) c[xi] = vel0 * double(Jq[0][xi]) + vel1 * double(Jq[1][xi]);
       double kp[ND];
-      double S = 0.0, SU = 0.0;
+      double S = 0.0, SU = 0.0, kU = 0.0;
 #pragma unroll
       for (int n = 0; n < ND; ++n) {
         double knt = double(0);
@@ -925,10 +944,19 @@ __device__ __forceinline__ void cell_residual(const double *__restrict__ tab, co
         kp[n] = fmax(kn, 0.0);
         lmax = fmax(lmax, fabs(kn));
         S += kp[n];
-        SU += kp[n] * Uq(n, 0);
+        if constexpr (NDIS) SU += kp[n] * Uq(n, 0);
+        if constexpr (LINF) kU += kn * Uq(n, 0);
       }
-      const double inv = 1.0 / S;
-      const double ub = SU * inv;
+      if constexpr (LINF) {
+        r[0] = kU;
+        if constexpr (PREC == 3 || PREC == 5) {
+#pragma unroll
+          for (int n = 0; n < ND; ++n) r[0] -= tab[O::V + q * ND + n] * nodal(n, 0);
+        }
+        fint[0] += wj * r[0];
+      }
+      const double inv = recip(S);
+      const double ub = NDIS ? SU * inv : 0.0;
       const double wr = wj * inv * r[0];
 #pragma unroll
       for (int n = 0; n < ND; ++n) {
@@ -1116,8 +1144,10 @@ __device__ __forceinline__ void cell_residual(const double *__restrict__ tab, co
 #pragma unroll 1
   for (int q = 0; q < NQ; ++q) {
     double r[M];
+    if constexpr (!LINF) {
 #pragma unroll
-    for (int k = 0; k < M; ++k) r[k] = lds_div[(q * M + k) * stride];
+      for (int k = 0; k < M; ++k) r[k] = lds_div[(q * M + k) * stride];
+    }
     if constexpr (AFFINE) {
       quad_point(q, r, Jinv[0], detJ[0]);
     } else {
@@ -1357,9 +1387,10 @@ struct PatchSize
 // floats.
 __host__ __device__ constexpr size_t patch_coff_doubles(int maxl) { return (static_cast<size_t>(maxl) + 3) / 4; }
 
-template <class PW, int M, int PREC>
+template <class PW, int PREC>
 __host__ __device__ constexpr size_t patch_lds_doubles(int maxl, int P)
 {
+  constexpr int M = PW::M;
   const size_t n = static_cast<size_t>(maxl);
   return n * M + patch_coff_doubles(maxl) + static_cast<size_t>(P) * PW::per_cell +
          (PREC == 2 ? n : (PREC == 3 ? n * M : (PREC == 4 ? (n * M + 1) / 2 : (PREC == 5 ? n * (M + 1) : 0))));
@@ -1400,8 +1431,8 @@ template <int M>
 __device__ __forceinline__ void node_step(const PatchArgs &a, uint32_t g, const double *acc, const double *u_old,
                                           double v, int di, double (&r)[M], double (&un)[M], double &d)
 {
-  const double iv = 1.0 / v;
-  d = a.lin_res ? a.lin_dt[g] : a.cfl * v / acc[M];
+  const double iv = recip(v);
+  d = a.lin_res ? a.lin_dt[g] : a.cfl * v * recip(acc[M]);
 #pragma unroll
   for (int k = 0; k < M; ++k) {
     const size_t j = static_cast<size_t>(g) * M + k;
@@ -1496,7 +1527,7 @@ __device__ __forceinline__ void patch_body(const PatchArgs &a, uint32_t pl, doub
 #pragma unroll
     for (int n = 0; n < ND; ++n) lc[n] = a.lconn[static_cast<size_t>(n) * a.ne + e];
   }
-  using PW = PatchWork<D, ND, NQ, AFFINE, M, SC, PREC>;
+  using PW = PatchWork<D, ND, NQ, AFFINE, PH, SC, PREC>;
   double *nodal_l = work + static_cast<size_t>(PATCH) * PW::per_cell;  // PREC 2, 3 and 5 only
   float *delta_l = reinterpret_cast<float *>(nodal_l);                 // PREC 4 only
   // (no global store before the cell work: the table loads stay scalar)

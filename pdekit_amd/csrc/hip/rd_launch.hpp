@@ -66,8 +66,7 @@ struct KernelSet
 template <int D, int NG, int ND, int NF, int NQ, bool AFF, int PH, int SC, int PREC = 0>
 hipError_t launch_cell(const CellArgs &a, unsigned grid, unsigned block, hipStream_t s)
 {
-  constexpr int M = PhysTraits<PH>::M;
-  const size_t lds = static_cast<size_t>(NQ) * M * block * sizeof(double);
+  const size_t lds = static_cast<size_t>(CellColumn<D, ND, NQ, AFF, PH>::value) * block * sizeof(double);
   hipLaunchKernelGGL((rd_cell_kernel<D, NG, ND, NF, NQ, AFF, PH, SC, PREC>), dim3(grid), dim3(block), lds, s, a);
   return hipGetLastError();
 }
@@ -75,9 +74,8 @@ hipError_t launch_cell(const CellArgs &a, unsigned grid, unsigned block, hipStre
 template <int D, int NG, int ND, int NF, int NQ, bool AFF, int PH, int SC, int PREC>
 hipError_t launch_patch(const PatchArgs &a, unsigned grid, int cells, hipStream_t s)
 {
-  constexpr int M = PhysTraits<PH>::M;
-  using PW = PatchWork<D, ND, NQ, AFF, M, SC, PREC>;
-  const size_t lds = patch_lds_doubles<PW, M, PREC>(a.maxl, cells) * sizeof(double);
+  using PW = PatchWork<D, ND, NQ, AFF, PH, SC, PREC>;
+  const size_t lds = patch_lds_doubles<PW, PREC>(a.maxl, cells) * sizeof(double);
   hipLaunchKernelGGL((rd_patch_kernel<D, NG, ND, NF, NQ, AFF, PH, SC, PREC>), dim3(grid), dim3(cells), lds, s, a);
   return hipGetLastError();
 }
@@ -109,16 +107,15 @@ hipError_t launch_jacobian(const JacArgs &a, unsigned grid, hipStream_t s)
   return hipGetLastError();
 }
 
-template <int D, int ND, int NQ, bool AFF, int M, int SC, int PREC>
+template <int D, int ND, int NQ, bool AFF, int PH, int SC, int PREC>
 size_t patch_lds_bytes(int maxl, int cells)
 {
-  return patch_lds_doubles<PatchWork<D, ND, NQ, AFF, M, SC, PREC>, M, PREC>(maxl, cells) * sizeof(double);
+  return patch_lds_doubles<PatchWork<D, ND, NQ, AFF, PH, SC, PREC>, PREC>(maxl, cells) * sizeof(double);
 }
 
 template <int D, int NG, int ND, int NF, int NQ, bool AFF, int PH, int SC>
 KernelSet kernel_set()
 {
-  constexpr int M = PhysTraits<PH>::M;
   KernelSet k;
   k.cell = &launch_cell<D, NG, ND, NF, NQ, AFF, PH, SC>;
   k.patch = &launch_patch<D, NG, ND, NF, NQ, AFF, PH, SC, 0>;
@@ -128,25 +125,25 @@ KernelSet kernel_set()
   // scalar ones)
   if constexpr ((PH == PH_ADVECTION2D || PH == PH_EULER2D || PH == PH_EULER3D) && SC == SC_LDA) {
     k.patch_lin = &launch_patch<D, NG, ND, NF, NQ, AFF, PH, SC, 4>;
-    k.patch_lin_lds_bytes = &patch_lds_bytes<D, ND, NQ, AFF, M, SC, 4>;
+    k.patch_lin_lds_bytes = &patch_lds_bytes<D, ND, NQ, AFF, PH, SC, 4>;
   }
   if constexpr (SC == SC_LDA || SC == SC_B) {
     k.cell_nodal = &launch_cell<D, NG, ND, NF, NQ, AFF, PH, SC, 2>;
     k.patch_nodal = &launch_patch<D, NG, ND, NF, NQ, AFF, PH, SC, 2>;
     k.patch_nodal_batch = &launch_patch_batch<D, NG, ND, NF, NQ, AFF, PH, SC, 2>;
-    k.patch_nodal_lds_bytes = &patch_lds_bytes<D, ND, NQ, AFF, M, SC, 2>;
+    k.patch_nodal_lds_bytes = &patch_lds_bytes<D, ND, NQ, AFF, PH, SC, 2>;
   }
   k.patch_src = &launch_patch<D, NG, ND, NF, NQ, AFF, PH, SC, 3>;
   k.patch_src_batch = &launch_patch_batch<D, NG, ND, NF, NQ, AFF, PH, SC, 3>;
   if constexpr (SC == SC_B) {
     k.patch_src_theta = &launch_patch<D, NG, ND, NF, NQ, AFF, PH, SC, 5>;
     k.patch_src_theta_batch = &launch_patch_batch<D, NG, ND, NF, NQ, AFF, PH, SC, 5>;
-    k.patch_src_theta_lds_bytes = &patch_lds_bytes<D, ND, NQ, AFF, M, SC, 5>;
+    k.patch_src_theta_lds_bytes = &patch_lds_bytes<D, ND, NQ, AFF, PH, SC, 5>;
   }
   if constexpr (SC != SC_PSI && SC != SC_BPSI) k.jacobian = &launch_jacobian<D, NG, ND, NF, NQ, AFF, PH, SC>;
-  k.patch_size = PatchSize<M, ND>::value;
-  k.patch_lds_bytes = &patch_lds_bytes<D, ND, NQ, AFF, M, SC, 0>;
-  k.patch_src_lds_bytes = &patch_lds_bytes<D, ND, NQ, AFF, M, SC, 3>;
+  k.patch_size = PatchSize<PhysTraits<PH>::M, ND>::value;
+  k.patch_lds_bytes = &patch_lds_bytes<D, ND, NQ, AFF, PH, SC, 0>;
+  k.patch_src_lds_bytes = &patch_lds_bytes<D, ND, NQ, AFF, PH, SC, 3>;
   return k;
 }
 

@@ -31,6 +31,14 @@ template <> struct PhysTraits<PH_BURGERS2D> { static constexpr int M = 1, DIM = 
 template <> struct PhysTraits<PH_EULER2D> { static constexpr int M = 4, DIM = 2; };
 template <> struct PhysTraits<PH_EULER3D> { static constexpr int M = 5, DIM = 3; };
 
+// Whether the P+1 flux element of a cell with ND nodes and NV vertices
+// interpolates the scalar flux exactly (its divergence is then a . grad u).
+template <int PH, int NV, int ND>
+struct ScalarFlux
+{
+  static constexpr bool exact = PH == PH_ADVECTION2D || PH == PH_ROTATION2D || (PH == PH_BURGERS2D && ND == NV);
+};
+
 struct PhysParams
 {
   double p0, p1;  // advection velocity (ax, ay) -- for PH_ROTATION2D the point's -- or (gamma, R)
