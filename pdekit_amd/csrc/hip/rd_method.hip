@@ -86,6 +86,15 @@ struct WeakDev
   double *d_qvel = nullptr;     // rotating advection: (y, -x) at every facet point
 };
 
+// A launch over weak boundary conditions of one facet kernel (launch_facets).
+struct WeakLaunch
+{
+  int key;
+  size_t args0, first0;
+  int count;
+  unsigned grid;
+};
+
 }  // namespace
 
 struct pdrd_method
@@ -105,6 +114,10 @@ struct pdrd_method
   int precision = 0;
   std::vector<WeakSpec> weak_specs;  // weak BCs added before pdrd_initialize
   std::vector<WeakDev> weak;
+  std::vector<WeakLaunch> weak_launches;
+  pdrd::WeakArgs *d_wargs = nullptr;  // [2][wargs_count], row buffers 0 and 1
+  uint32_t *d_wfirst = nullptr;
+  size_t wargs_count = 0;
   // mixed precision (linearised defect correction). An FP64 sweep sets the
   // linearisation point: u_ref = u, its FP64 residual in d_res and time step
   // in d_dt; every `refresh` iterations it also recomputes the element
@@ -564,56 +577,114 @@ int launch_patch_blocks(pdrd_method *h, int update, int outputs, int excl, doubl
   return PDRD_OK;
 }
 
+// Arguments of a method's weak boundary condition w, rows into row buffer
+// `buffer`.
+pdrd::WeakArgs weak_args(const pdrd_method *h, const WeakDev &w, int buffer)
+{
+  pdrd::WeakArgs a{};
+  a.nodes = w.d_nodes;
+  a.rows = w.d_rows;
+  a.normal = w.d_normal;
+  a.jac = w.d_jac;
+  a.w = w.d_w;
+  a.V = w.d_V;
+  a.u = h->d_u;
+  a.vol = h->d_vol;
+  a.slot_acc = rows_buffer(h, buffer);
+  a.status = h->d_status;
+  a.nf = w.nf;
+  a.nq = w.nq;
+  a.type = w.type;
+  a.relax = w.relax;
+  a.qstate = w.d_qstate;
+  a.qvel = w.d_qvel;
+  for (int i = 0; i < 5; ++i) a.params[i] = w.params[i];
+  a.pp.p0 = h->params[0];
+  a.pp.p1 = h->params[1];
+  return a;
+}
+
+uint32_t weak_blocks(const WeakDev &w) { return (w.nf + pdrd::WEAK_THREADS - 1) / pdrd::WEAK_THREADS; }
+
+int weak_key(int physics, int nfn) { return physics * 8 + nfn; }
+
+// One launch of facet kernel `key`: `count` conditions with their workgroup
+// prefix sums, `grid` workgroups.
+int launch_facets(int key, const pdrd::WeakArgs *w, const uint32_t *first, int count, unsigned grid, hipStream_t s)
+{
+#define WEAK_CASE(PH, NFN)                                                                                   \
+  case PH * 8 + NFN:                                                                                         \
+    hipLaunchKernelGGL((pdrd::weak_bc_kernel<PH, NFN>), dim3(grid), dim3(pdrd::WEAK_THREADS), 0, s, w, first, \
+                       count);                                                                               \
+    break;
+  switch (key) {
+    WEAK_CASE(pdrd::PH_ADVECTION2D, 2)
+    WEAK_CASE(pdrd::PH_ADVECTION2D, 3)
+    WEAK_CASE(pdrd::PH_BURGERS2D, 2)
+    WEAK_CASE(pdrd::PH_BURGERS2D, 3)
+    WEAK_CASE(pdrd::PH_ROTATION2D, 2)
+    WEAK_CASE(pdrd::PH_ROTATION2D, 3)
+    WEAK_CASE(pdrd::PH_EULER2D, 2)
+    WEAK_CASE(pdrd::PH_EULER2D, 3)
+    WEAK_CASE(pdrd::PH_EULER3D, 3)
+    WEAK_CASE(pdrd::PH_EULER3D, 6)
+    default: return set_error(PDRD_ENOTSUP, "weak boundary condition on this facet kind");
+  }
+#undef WEAK_CASE
+  HIP_CHECK(hipGetLastError());
+  return PDRD_OK;
+}
+
+// The method's weak boundary conditions as its own sweeps launch them: grouped
+// by facet kernel, arguments for row buffers 0 and 1 (h->d_wargs) and prefix
+// sums (h->d_wfirst). Called when the conditions or their device arrays
+// change.
+int upload_weak(pdrd_method *h)
+{
+  h->weak_launches.clear();
+  std::vector<pdrd::WeakArgs> args[2];
+  std::vector<uint32_t> first;
+  for (const WeakDev &w : h->weak)
+    if (w.nf) {
+      const int key = weak_key(h->physics, w.nfn);
+      bool known = false;
+      for (const WeakLaunch &l : h->weak_launches) known = known || l.key == key;
+      if (!known) h->weak_launches.push_back(WeakLaunch{key, 0, 0, 0, 0});
+    }
+  for (WeakLaunch &l : h->weak_launches) {
+    l.args0 = args[0].size();
+    l.first0 = first.size();
+    first.push_back(0);
+    for (const WeakDev &w : h->weak) {
+      if (w.nf == 0 || weak_key(h->physics, w.nfn) != l.key) continue;
+      for (int i = 0; i < 2; ++i) args[i].push_back(weak_args(h, w, i));
+      l.grid += weak_blocks(w);
+      first.push_back(l.grid);
+      ++l.count;
+    }
+  }
+  h->wargs_count = args[0].size();
+  if (args[0].empty()) return PDRD_OK;
+  args[0].insert(args[0].end(), args[1].begin(), args[1].end());
+  if (!h->d_wargs) {
+    if (int rc = dev_alloc(h, &h->d_wargs, args[0].size())) return rc;
+    if (int rc = dev_alloc(h, &h->d_wfirst, first.size())) return rc;
+  }
+  HIP_CHECK(hipMemcpy(h->d_wargs, args[0].data(), args[0].size() * sizeof(pdrd::WeakArgs), hipMemcpyHostToDevice));
+  HIP_CHECK(hipMemcpy(h->d_wfirst, first.data(), first.size() * sizeof(uint32_t), hipMemcpyHostToDevice));
+  return PDRD_OK;
+}
+
 // The weak boundary conditions' facet kernels: after the patch kernels of a
 // sweep (whose facet nodes are all shared, so u holds their state at the
 // sweep's start) and before the shared-node sums; rows into row buffer
 // `buffer`.
 int launch_weak(pdrd_method *h, hipStream_t s, int buffer = 0)
 {
-  for (const WeakDev &w : h->weak) {
-    if (w.nf == 0) continue;
-    pdrd::WeakArgs a{};
-    a.nodes = w.d_nodes;
-    a.rows = w.d_rows;
-    a.normal = w.d_normal;
-    a.jac = w.d_jac;
-    a.w = w.d_w;
-    a.V = w.d_V;
-    a.u = h->d_u;
-    a.vol = h->d_vol;
-    a.slot_acc = rows_buffer(h, buffer);
-    a.status = h->d_status;
-    a.nf = w.nf;
-    a.nq = w.nq;
-    a.type = w.type;
-    a.relax = w.relax;
-    a.qstate = w.d_qstate;
-    a.qvel = w.d_qvel;
-    for (int i = 0; i < 5; ++i) a.params[i] = w.params[i];
-    a.pp.p0 = h->params[0];
-    a.pp.p1 = h->params[1];
-    const dim3 grid((w.nf + 127) / 128);
-    const int key = h->physics * 8 + w.nfn;
-#define WEAK_CASE(PH, NFN)                                                                   \
-  case PH * 8 + NFN:                                                                         \
-    hipLaunchKernelGGL((pdrd::weak_bc_kernel<PH, NFN>), grid, dim3(128), 0, s, a);           \
-    break;
-    switch (key) {
-      WEAK_CASE(pdrd::PH_ADVECTION2D, 2)
-      WEAK_CASE(pdrd::PH_ADVECTION2D, 3)
-      WEAK_CASE(pdrd::PH_BURGERS2D, 2)
-      WEAK_CASE(pdrd::PH_BURGERS2D, 3)
-      WEAK_CASE(pdrd::PH_ROTATION2D, 2)
-      WEAK_CASE(pdrd::PH_ROTATION2D, 3)
-      WEAK_CASE(pdrd::PH_EULER2D, 2)
-      WEAK_CASE(pdrd::PH_EULER2D, 3)
-      WEAK_CASE(pdrd::PH_EULER3D, 3)
-      WEAK_CASE(pdrd::PH_EULER3D, 6)
-      default: return set_error(PDRD_ENOTSUP, "weak boundary condition on this facet kind");
-    }
-#undef WEAK_CASE
-    HIP_CHECK(hipGetLastError());
-  }
+  for (const WeakLaunch &l : h->weak_launches)
+    if (int rc = launch_facets(l.key, h->d_wargs + buffer * h->wargs_count + l.args0, h->d_wfirst + l.first0, l.count,
+                               l.grid, s))
+      return rc;
   return PDRD_OK;
 }
 
@@ -841,6 +912,11 @@ void free_device(pdrd_method *h)
     (void)hipFree(w.d_qvel);
   }
   h->weak.clear();
+  h->weak_launches.clear();
+  (void)hipFree(h->d_wargs);
+  (void)hipFree(h->d_wfirst);
+  h->d_wargs = nullptr;
+  h->d_wfirst = nullptr;
   (void)hipFree(h->d_pn_coff);
   (void)hipFree(h->d_slot_acc);
   (void)hipFree(h->d_patch_partial);
@@ -1467,6 +1543,7 @@ int pdrd_initialize(pdrd_method_t h)
     h->own_stream = true;
   }
   for (hipEvent_t &e : h->ev) HIP_CHECK(hipEventCreate(&e));
+  if ((rc = upload_weak(h))) { free_device(h); return rc; }
   HIP_CHECK(hipDeviceSynchronize());
   h->ready = true;
   return PDRD_OK;
@@ -1650,16 +1727,25 @@ int pdrd_set_weak_bc_state(pdrd_method_t h, int k, const double *state, size_t c
   WeakDev &w = h->weak[k];
   if (w.type != PDRD_WEAK_DIRICHLET) return set_error(PDRD_ENOTSUP, "point states are for WeakDirichlet");
   if (!state) {
+    if (!w.d_qstate) return PDRD_OK;
+    HIP_CHECK(hipStreamSynchronize(h->stream));
     (void)hipFree(w.d_qstate);
     w.d_qstate = nullptr;
-    return PDRD_OK;
+    return upload_weak(h);
   }
   const size_t n = static_cast<size_t>(w.nf) * w.nq * h->m;
   if (count != n)
     return set_error(PDRD_EINVAL, "state holds " + std::to_string(count) + " values, the facet points need " +
                                       std::to_string(n) + " ([facets][points][m])");
-  if (!w.d_qstate)
+  if (!w.d_qstate) {
+    HIP_CHECK(hipStreamSynchronize(h->stream));
     if (int rc = dev_alloc(h, &w.d_qstate, n)) return rc;
+    if (int rc = upload_weak(h)) {
+      (void)hipFree(w.d_qstate);
+      w.d_qstate = nullptr;
+      return rc;
+    }
+  }
   HIP_CHECK(hipMemcpyAsync(w.d_qstate, state, n * sizeof(double), hipMemcpyHostToDevice, h->stream));
   HIP_CHECK(hipStreamSynchronize(h->stream));
   return PDRD_OK;
@@ -2175,8 +2261,9 @@ struct pdrd_batch
   hipStream_t stream = nullptr;
   pdrd::PatchArgs *d_pargs = nullptr;
   pdrd::FixupArgs *d_fargs = nullptr;
+  pdrd::WeakArgs *d_wargs = nullptr;
   uint32_t *d_first = nullptr;
-  size_t pargs_cap = 0, fargs_cap = 0, first_cap = 0;
+  size_t pargs_cap = 0, fargs_cap = 0, wargs_cap = 0, first_cap = 0;
   int graphs = 0;  // 1: replay the iterations of a call from a captured HIP graph
 };
 
@@ -2201,6 +2288,7 @@ struct BatchLaunch
 {
   pdrd::PatchBatchLauncher patch = nullptr;  // null: shared-node sums
   int m = 0;                                 // equations (shared-node sums)
+  int weak_key = -1;                         // facet kernel (weak boundary conditions)
   int cells = 0;                             // threads per workgroup of a patch launch
   size_t args0 = 0, first0 = 0;              // offsets in the argument / prefix arrays
   int count = 0;
@@ -2250,16 +2338,19 @@ KindPlace kind_place(int kind, bool chain)
 // One batched sweep of kind `kind`: the patch launches (arguments of the kind
 // at kind * args_per_kind), the weak facet kernels of every method, the
 // shared-node sums of the methods that close in this kind.
-int enqueue_batch(pdrd_batch *b, const std::vector<BatchLaunch> &patches, const std::vector<BatchLaunch> &fixups,
-                  size_t args_per_kind, int kind, int count, const pdrd_method_t *methods, const bool *chain)
+int enqueue_batch(pdrd_batch *b, const std::vector<BatchLaunch> &patches, const std::vector<BatchLaunch> &weak,
+                  const std::vector<BatchLaunch> &fixups, size_t pargs_per_kind, size_t wargs_per_kind, int kind)
 {
   for (const BatchLaunch &l : patches) {
     if (l.grid == 0) continue;
-    HIP_CHECK(l.patch(b->d_pargs + kind * args_per_kind + l.args0, b->d_first + l.first0, l.count, l.grid, l.cells,
+    HIP_CHECK(l.patch(b->d_pargs + kind * pargs_per_kind + l.args0, b->d_first + l.first0, l.count, l.grid, l.cells,
                       l.lds, b->stream));
   }
-  for (int i = 0; i < count; ++i)
-    if (int rc = launch_weak(methods[i], b->stream, kind_place(kind, chain[i]).c.write)) return rc;
+  for (const BatchLaunch &l : weak) {
+    if (int rc = launch_facets(l.weak_key, b->d_wargs + kind * wargs_per_kind + l.args0, b->d_first + l.first0, l.count,
+                               l.grid, b->stream))
+      return rc;
+  }
   for (const BatchLaunch &l : fixups) {
     if (l.grid == 0) continue;
     const pdrd::FixupArgs *fa = b->d_fargs + l.args0;
@@ -2306,6 +2397,7 @@ int pdrd_batch_destroy(pdrd_batch_t b)
   (void)hipStreamSynchronize(b->stream);
   (void)hipFree(b->d_pargs);
   (void)hipFree(b->d_fargs);
+  (void)hipFree(b->d_wargs);
   (void)hipFree(b->d_first);
   (void)hipStreamDestroy(b->stream);
   delete b;
@@ -2394,6 +2486,47 @@ int pdrd_batch_iterate(pdrd_batch_t b, int count, const pdrd_method_t *methods, 
   }
   const size_t ph = pk[0].size();
   for (int k = 0; k < BK_COUNT; ++k) pargs.insert(pargs.end(), pk[k].begin(), pk[k].end());
+  // weak facets of every kind: one launch per facet kernel over the conditions
+  // of all methods
+  std::vector<BatchLaunch> weak;
+  std::vector<pdrd::WeakArgs> wk[BK_COUNT];
+  {
+    std::vector<std::vector<std::pair<int, size_t>>> wmembers;  // (method, condition) per launch
+    for (int i = 0; i < count; ++i)
+      for (size_t k = 0; k < methods[i]->weak.size(); ++k) {
+        const WeakDev &w = methods[i]->weak[k];
+        if (w.nf == 0) continue;
+        const int key = weak_key(methods[i]->physics, w.nfn);
+        size_t g = 0;
+        while (g < weak.size() && weak[g].weak_key != key) ++g;
+        if (g == weak.size()) {
+          BatchLaunch l;
+          l.weak_key = key;
+          weak.push_back(l);
+          wmembers.emplace_back();
+        }
+        wmembers[g].emplace_back(i, k);
+      }
+    for (size_t g = 0; g < weak.size(); ++g) {
+      BatchLaunch &l = weak[g];
+      l.first0 = first.size();
+      l.args0 = wk[0].size();
+      l.count = static_cast<int>(wmembers[g].size());
+      uint32_t acc = 0;
+      first.push_back(0);
+      for (const auto &mk : wmembers[g]) {
+        const WeakDev &w = methods[mk.first]->weak[mk.second];
+        for (int k = 0; k < BK_COUNT; ++k)
+          wk[k].push_back(weak_args(methods[mk.first], w, kind_place(k, chain[mk.first]).c.write));
+        acc += weak_blocks(w);
+        first.push_back(acc);
+      }
+      l.grid = acc;
+    }
+  }
+  const size_t wh = wk[0].size();
+  std::vector<pdrd::WeakArgs> wargs;
+  for (int k = 0; k < BK_COUNT; ++k) wargs.insert(wargs.end(), wk[k].begin(), wk[k].end());
   // shared-node sums of every kind: one launch per number of equations over
   // the methods that close in that kind
   std::vector<BatchLaunch> fixups[BK_COUNT];
@@ -2424,14 +2557,17 @@ int pdrd_batch_iterate(pdrd_batch_t b, int count, const pdrd_method_t *methods, 
     }
   if (int rc = grow(&b->d_pargs, &b->pargs_cap, pargs.size())) return rc;
   if (int rc = grow(&b->d_fargs, &b->fargs_cap, fargs.size())) return rc;
+  if (int rc = grow(&b->d_wargs, &b->wargs_cap, wargs.size())) return rc;
   if (int rc = grow(&b->d_first, &b->first_cap, first.size())) return rc;
+  if (!wargs.empty())
+    HIP_CHECK(hipMemcpy(b->d_wargs, wargs.data(), wargs.size() * sizeof(pdrd::WeakArgs), hipMemcpyHostToDevice));
   if (!pargs.empty())
     HIP_CHECK(hipMemcpy(b->d_pargs, pargs.data(), pargs.size() * sizeof(pdrd::PatchArgs), hipMemcpyHostToDevice));
   if (!fargs.empty())
     HIP_CHECK(hipMemcpy(b->d_fargs, fargs.data(), fargs.size() * sizeof(pdrd::FixupArgs), hipMemcpyHostToDevice));
   HIP_CHECK(hipMemcpy(b->d_first, first.data(), first.size() * sizeof(uint32_t), hipMemcpyHostToDevice));
 
-  auto sweep = [&](int kind) { return enqueue_batch(b, patches, fixups[kind], ph, kind, count, methods, chain); };
+  auto sweep = [&](int kind) { return enqueue_batch(b, patches, weak, fixups[kind], ph, wh, kind); };
   if (n_iter == 1) {
     if (int rc = sweep(BK_SINGLE)) return rc;
   } else if (!b->graphs) {

@@ -5,7 +5,7 @@
 // WeakSuperInlet.hpp, WeakDirichlet.hpp over WeakBC::apply,
 // WeakBC.hpp:225-352, 786-821).
 //
-// One thread per facet. Per facet quadrature point q (state u_q = V u):
+// One thread per facet (weak_facet). Per facet quadrature point q (state u_q = V u):
 //   WeakWall:       dF = F(u_g) n - F(u_q) n, u_g = u_q without its normal
 //                   velocity (same density and pressure);
 //   WeakSuperInlet: dF = 0 (only the wave speed is added);
@@ -178,12 +178,11 @@ __device__ __forceinline__ double weak_point(const WeakArgs &a, const double *uq
   }
 }
 
+// One facet of one condition.
 template <int PH, int NFN>
-__global__ __launch_bounds__(128) void weak_bc_kernel(WeakArgs a)
+__device__ __forceinline__ void weak_facet(const WeakArgs &a, uint32_t f)
 {
   constexpr int D = PhysTraits<PH>::DIM, M = PhysTraits<PH>::M;
-  const uint32_t f = blockIdx.x * blockDim.x + threadIdx.x;
-  if (f >= a.nf) return;
   double U[NFN][M];
   uint32_t nid[NFN];
 #pragma unroll
@@ -247,6 +246,26 @@ __global__ __launch_bounds__(128) void weak_bc_kernel(WeakArgs a)
     row[M] = a.vol[nid[n]] * coeff;
   }
   if (bad) atomicOr(a.status, 1);
+}
+
+// The conditions of one launch (device arrays): workgroup g runs facets of
+// condition i, first[i] <= g < first[i + 1]. All conditions of a method, or of
+// all methods of a batch, go in one launch: the few hundred facets of one
+// condition take 5 us, nearly all of it latency, and four of them in a row were
+// a quarter of a 66 us sweep of the bump channel, 13 of them a quarter of a
+// serving batch's. (As a kernel argument by value the conditions, indexed by
+// workgroup, would be copied to scratch memory.)
+constexpr unsigned WEAK_THREADS = 64;
+
+template <int PH, int NFN>
+__global__ __launch_bounds__(WEAK_THREADS) void weak_bc_kernel(const WeakArgs *__restrict__ w,
+                                                               const uint32_t *__restrict__ first, int count)
+{
+  const uint32_t g = blockIdx.x;
+  int i = 0;
+  while (i + 1 < count && first[i + 1] <= g) ++i;
+  const uint32_t f = (g - first[i]) * WEAK_THREADS + threadIdx.x;
+  if (f < w[i].nf) weak_facet<PH, NFN>(w[i], f);
 }
 
 }  // namespace pdrd
