@@ -339,7 +339,8 @@ int pdrd_last_timing(pdrd_method_t h, double *cell_ms, double *node_ms);
  * methods, with the patches of every method of one element type / physics /
  * scheme in one launch per iteration and the shared-node sums of every method
  * with the same number of equations in another, launched directly on the
- * batch's stream (or, after pdrd_batch_set_graphs(b, 1), captured once per
+ * batch's streams, one for each group of methods that share launches and at
+ * most four (or, after pdrd_batch_set_graphs(b, 1), captured once per
  * call into a HIP graph replayed for all but the last iteration: measured
  * slower on MI355X, whose direct launches cost less than the replays; p99 of
  * the serving stream 2.67 s direct against 2.87 s from graphs). Each method advances
