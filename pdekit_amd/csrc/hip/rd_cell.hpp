@@ -78,12 +78,13 @@ struct TabOffsets
 // Workgroups are dealt round-robin to the 8 XCDs; give each XCD one
 // contiguous range of workgroups so neighbouring cells (which share nodes)
 // meet in the same L2.
-__device__ __forceinline__ uint32_t xcd_block_index()
+__device__ __forceinline__ uint32_t xcd_block_index(uint32_t bid, uint32_t nb)
 {
-  const uint32_t nb = gridDim.x, bid = blockIdx.x;
   const uint32_t x = bid & 7u, k = bid >> 3, q8 = nb >> 3, r8 = nb & 7u;
   return x * q8 + (x < r8 ? x : r8) + k;
 }
+
+__device__ __forceinline__ uint32_t xcd_block_index() { return xcd_block_index(blockIdx.x, gridDim.x); }
 
 __device__ __forceinline__ void scatter_add(double *p, double v, int atomic)
 {

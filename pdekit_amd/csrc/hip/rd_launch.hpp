@@ -5,6 +5,7 @@
 
 #include "rd_cell.hpp"
 #include "rd_jacobian.hpp"
+#include "rd_weakbc.hpp"
 
 namespace pdrd {
 
@@ -12,6 +13,10 @@ using CellLauncher = hipError_t (*)(const CellArgs &, unsigned grid, unsigned bl
 using PatchLauncher = hipError_t (*)(const PatchArgs &, unsigned grid, int cells, hipStream_t);
 using PatchBatchLauncher = hipError_t (*)(const PatchArgs *args, const uint32_t *first, int count, unsigned grid,
                                           int cells, size_t lds_bytes, hipStream_t);
+// quad, tri: the two blocks; weak: the facets of the method's weak boundary
+// conditions (groups of 64; weak_groups 0: none)
+using PatchMixedLauncher = hipError_t (*)(const PatchArgs &quad, const PatchArgs &tri, const WeakRange &weak,
+                                          unsigned weak_groups, int cells, hipStream_t);
 using JacobianLauncher = hipError_t (*)(const JacArgs &, unsigned grid, hipStream_t);
 
 struct CellKey
@@ -29,6 +34,9 @@ struct KernelSet
   PatchBatchLauncher patch_nodal_batch = nullptr;
   PatchBatchLauncher patch_src_batch = nullptr;
   PatchLauncher patch_lin = nullptr;  // linear sweep of the mixed-precision form: J delta per cell
+  // first-order quadrilaterals of the 2D Euler equations: with the triangles
+  // of the same mesh and the weak facets in one launch
+  PatchMixedLauncher patch_mixed = nullptr;
   // with the nodal input of the scheme (LDA: artificial viscosity, B:
   // external blending coefficient); null for N and PSI, which take none
   CellLauncher cell_nodal = nullptr;
@@ -80,6 +88,41 @@ hipError_t launch_patch(const PatchArgs &a, unsigned grid, int cells, hipStream_
   return hipGetLastError();
 }
 
+// A sweep of a mixed mesh of first-order quadrilaterals and triangles of the 2D
+// Euler equations in one launch: workgroups [0, quad.np) take the
+// quadrilaterals' patches, the next tri.np the triangles', the rest the weak
+// facets (64 to a wave), all of which only read the state of shared nodes. One
+// after the other, each kind fills the chip for a round or two and then drains
+// it: 65 536 + 131 072 cells LDA 30.6 + 16.8 us, and 5 us of facets.
+template <int SC>
+__global__ __launch_bounds__(128, 2) void rd_patch_mixed_kernel(PatchArgs quad, PatchArgs tri, WeakRange weak,
+                                                                uint32_t weak_groups)
+{
+  extern __shared__ double lds[];
+  const uint32_t g = blockIdx.x;
+  if (g < quad.np) {
+    patch_body<2, 4, 4, 9, 8, false, PH_EULER2D, SC, 0>(quad, xcd_block_index(g, quad.np), lds);
+  } else if (g < quad.np + tri.np) {
+    patch_body<2, 3, 3, 6, 6, true, PH_EULER2D, SC, 0>(tri, xcd_block_index(g - quad.np, tri.np), lds);
+  } else {
+    const uint32_t w = (g - quad.np - tri.np) * (blockDim.x / WEAK_THREADS) + threadIdx.x / WEAK_THREADS;
+    if (w < weak_groups) weak_group<PH_EULER2D, 2>(weak, w, threadIdx.x % WEAK_THREADS);
+  }
+}
+
+template <int SC>
+hipError_t launch_patch_mixed(const PatchArgs &quad, const PatchArgs &tri, const WeakRange &weak, unsigned weak_groups,
+                              int cells, hipStream_t s)
+{
+  const size_t lq = patch_lds_doubles<PatchWork<2, 4, 8, false, PH_EULER2D, SC, 0>, 0>(quad.maxl, cells);
+  const size_t lt = patch_lds_doubles<PatchWork<2, 3, 6, true, PH_EULER2D, SC, 0>, 0>(tri.maxl, cells);
+  const unsigned waves = cells / WEAK_THREADS;
+  const unsigned grid = quad.np + tri.np + (weak_groups + waves - 1) / waves;
+  hipLaunchKernelGGL((rd_patch_mixed_kernel<SC>), dim3(grid), dim3(cells), (lq > lt ? lq : lt) * sizeof(double), s, quad,
+                     tri, weak, weak_groups);
+  return hipGetLastError();
+}
+
 template <int D, int NG, int ND, int NF, int NQ, bool AFF, int PH, int SC, int PREC>
 hipError_t launch_patch_batch(const PatchArgs *args, const uint32_t *first, int count, unsigned grid, int cells,
                               size_t lds, hipStream_t s)
@@ -127,6 +170,7 @@ KernelSet kernel_set()
     k.patch_lin = &launch_patch<D, NG, ND, NF, NQ, AFF, PH, SC, 4>;
     k.patch_lin_lds_bytes = &patch_lds_bytes<D, ND, NQ, AFF, PH, SC, 4>;
   }
+  if constexpr (PH == PH_EULER2D && !AFF && ND == 4 && NQ == 8) k.patch_mixed = &launch_patch_mixed<SC>;
   if constexpr (SC == SC_LDA || SC == SC_B) {
     k.cell_nodal = &launch_cell<D, NG, ND, NF, NQ, AFF, PH, SC, 2>;
     k.patch_nodal = &launch_patch<D, NG, ND, NF, NQ, AFF, PH, SC, 2>;

@@ -614,8 +614,8 @@ int launch_facets(int key, const pdrd::WeakArgs *w, const uint32_t *first, int c
 {
 #define WEAK_CASE(PH, NFN)                                                                                   \
   case PH * 8 + NFN:                                                                                         \
-    hipLaunchKernelGGL((pdrd::weak_bc_kernel<PH, NFN>), dim3(grid), dim3(pdrd::WEAK_THREADS), 0, s, w, first, \
-                       count);                                                                               \
+    hipLaunchKernelGGL((pdrd::weak_bc_kernel<PH, NFN>), dim3(grid), dim3(pdrd::WEAK_THREADS), 0, s,          \
+                       pdrd::WeakRange{w, first, count});                                                    \
     break;
   switch (key) {
     WEAK_CASE(pdrd::PH_ADVECTION2D, 2)
@@ -710,14 +710,52 @@ int launch_fixup(pdrd_method *h, int update, int outputs, int excl, double cfl, 
   return PDRD_OK;
 }
 
+// The quadrilateral and the triangle block of a method whose sweeps go in one
+// launch (KernelSet::patch_mixed): a mixed first-order mesh of the 2D Euler
+// equations without nodal inputs, both blocks with the same cells per patch,
+// and no weak conditions on another kind of facet.
+bool mixed_launch(const pdrd_method *h, const Block **quad, const Block **tri)
+{
+  if (h->physics != PDRD_EULER2D || h->blocks.size() != 2 || h->use_src || nodal_input(h)) return false;
+  const Block &a = h->blocks[0], &b = h->blocks[1];
+  *quad = a.ks.patch_mixed ? &a : &b;
+  *tri = a.ks.patch_mixed ? &b : &a;
+  const pdrd_fe_desc &t = (*tri)->fe;
+  return (*quad)->ks.patch_mixed && t.shape == PDRD_TRIAG && t.sol_order == 1 && t.nq == 6 && a.cells == b.cells &&
+         a.np && b.np && h->weak_launches.size() <= 1;
+}
+
+// The patch and facet kernels of one sweep: weak facets read the state at the
+// sweep's start, which u holds during the patch kernels unless the sweep's own
+// patches finish the previous one's shared nodes (c.pend).
+int launch_sweep_cells(pdrd_method *h, int update, int outputs, int excl, double cfl, Chain c = {}, bool lin = false)
+{
+  const Block *quad, *tri;
+  if (!lin && mixed_launch(h, &quad, &tri)) {
+    const bool with_weak = c.pend < 0 && !h->weak_launches.empty();
+    pdrd::WeakRange w{};
+    unsigned groups = 0;
+    if (with_weak) {
+      const WeakLaunch &l = h->weak_launches[0];
+      w = pdrd::WeakRange{h->d_wargs + c.write * h->wargs_count + l.args0, h->d_wfirst + l.first0, l.count};
+      groups = l.grid;
+    }
+    HIP_CHECK(quad->ks.patch_mixed(patch_args(h, quad, update, outputs, excl, cfl, c),
+                                   patch_args(h, tri, update, outputs, excl, cfl, c), w, groups, quad->cells,
+                                   h->stream));
+    return with_weak ? PDRD_OK : launch_weak(h, h->stream, c.write);
+  }
+  if (int rc = launch_patch_blocks(h, update, outputs, excl, cfl, c, lin)) return rc;
+  return launch_weak(h, h->stream, c.write);
+}
+
 // Patch assembly of every block followed by the sums of the shared nodes.
 // update = 0: residual and wave speed of every node; update = 1: one
 // pseudo-time iteration (the strong Dirichlet values are applied in the
 // nodal step), with res / dt / ws / norm partials when outputs is set.
 int launch_patches(pdrd_method *h, int update, int outputs, int excl, double cfl)
 {
-  if (int rc = launch_patch_blocks(h, update, outputs, excl, cfl)) return rc;
-  if (int rc = launch_weak(h, h->stream)) return rc;
+  if (int rc = launch_sweep_cells(h, update, outputs, excl, cfl)) return rc;
   return launch_fixup(h, update, outputs, excl, cfl);
 }
 
@@ -727,8 +765,7 @@ int launch_patches(pdrd_method *h, int update, int outputs, int excl, double cfl
 // next sweep.
 int launch_chain_sweep(pdrd_method *h, int outputs, int excl, double cfl, Chain c, bool close, bool lin = false)
 {
-  if (int rc = launch_patch_blocks(h, 1, outputs, excl, cfl, c, lin)) return rc;
-  if (int rc = launch_weak(h, h->stream, c.write)) return rc;
+  if (int rc = launch_sweep_cells(h, 1, outputs, excl, cfl, c, lin)) return rc;
   return close ? launch_fixup(h, 1, outputs, excl, cfl, c.write, lin) : PDRD_OK;
 }
 
@@ -1061,8 +1098,8 @@ int iterate_norm(pdrd_method *h, double *norm)
 // launched directly: replaying them from captured HIP graphs measured slower
 // on MI355X (25.6 against 11.1 us per sweep of a 32 768-cell P1 mesh, the
 // launches being dearer than the kernels). With timing on, events bracket the
-// patch kernels (cell interval) and the facet kernels + fix-up (node
-// interval) of every sweep.
+// patch and facet kernels (cell interval) and the fix-up (node interval) of
+// every sweep.
 // Default: chained for the scalar physics (fewer launches, little shared-node
 // work per patch), not for the Euler systems, whose patches hold more shared
 // nodes of more equations, so that the deferred steps cost more in their
@@ -1107,9 +1144,8 @@ int iterate_patches(pdrd_method *h, double cfl, int n_iter, int excl, double *no
     c.record = !close;
     if (h->timing) {
       HIP_CHECK(hipEventRecord(h->ev[0], h->stream));
-      if (int rc = launch_patch_blocks(h, 1, out, excl, cfl, c, lin)) return rc;
+      if (int rc = launch_sweep_cells(h, 1, out, excl, cfl, c, lin)) return rc;
       HIP_CHECK(hipEventRecord(h->ev[1], h->stream));
-      if (int rc = launch_weak(h, h->stream, c.write)) return rc;
       if (close)
         if (int rc = launch_fixup(h, 1, out, excl, cfl, c.write, lin)) return rc;
       HIP_CHECK(hipEventRecord(h->ev[2], h->stream));

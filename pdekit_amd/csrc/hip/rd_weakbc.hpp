@@ -257,15 +257,27 @@ __device__ __forceinline__ void weak_facet(const WeakArgs &a, uint32_t f)
 // workgroup, would be copied to scratch memory.)
 constexpr unsigned WEAK_THREADS = 64;
 
-template <int PH, int NFN>
-__global__ __launch_bounds__(WEAK_THREADS) void weak_bc_kernel(const WeakArgs *__restrict__ w,
-                                                               const uint32_t *__restrict__ first, int count)
+struct WeakRange
 {
-  const uint32_t g = blockIdx.x;
+  const WeakArgs *w;
+  const uint32_t *first;  // workgroup (64 facets) prefix sums, [count + 1]
+  int count;
+};
+
+// Facet `lane` of workgroup g of the range.
+template <int PH, int NFN>
+__device__ __forceinline__ void weak_group(const WeakRange &r, uint32_t g, uint32_t lane)
+{
   int i = 0;
-  while (i + 1 < count && first[i + 1] <= g) ++i;
-  const uint32_t f = (g - first[i]) * WEAK_THREADS + threadIdx.x;
-  if (f < w[i].nf) weak_facet<PH, NFN>(w[i], f);
+  while (i + 1 < r.count && r.first[i + 1] <= g) ++i;
+  const uint32_t f = (g - r.first[i]) * WEAK_THREADS + lane;
+  if (f < r.w[i].nf) weak_facet<PH, NFN>(r.w[i], f);
+}
+
+template <int PH, int NFN>
+__global__ __launch_bounds__(WEAK_THREADS) void weak_bc_kernel(WeakRange r)
+{
+  weak_group<PH, NFN>(r, blockIdx.x, threadIdx.x);
 }
 
 }  // namespace pdrd
