@@ -17,6 +17,11 @@ using PatchBatchLauncher = hipError_t (*)(const PatchArgs *args, const uint32_t 
 // conditions (groups of 64; weak_groups 0: none)
 using PatchMixedLauncher = hipError_t (*)(const PatchArgs &quad, const PatchArgs &tri, const WeakRange &weak,
                                           unsigned weak_groups, int cells, hipStream_t);
+// The same over `count` methods: args [2][count] (quadrilaterals, triangles) and
+// the prefix sums of their patches first [2][count + 1], grids nq and nt.
+using PatchMixedBatchLauncher = hipError_t (*)(const PatchArgs *args, const uint32_t *first, int count, unsigned nq,
+                                               unsigned nt, const WeakRange &weak, unsigned weak_groups, int cells,
+                                               size_t lds, hipStream_t);
 using JacobianLauncher = hipError_t (*)(const JacArgs &, unsigned grid, hipStream_t);
 
 struct CellKey
@@ -37,6 +42,7 @@ struct KernelSet
   // first-order quadrilaterals of the 2D Euler equations: with the triangles
   // of the same mesh and the weak facets in one launch
   PatchMixedLauncher patch_mixed = nullptr;
+  PatchMixedBatchLauncher patch_mixed_batch = nullptr;
   // with the nodal input of the scheme (LDA: artificial viscosity, B:
   // external blending coefficient); null for N and PSI, which take none
   CellLauncher cell_nodal = nullptr;
@@ -111,6 +117,44 @@ __global__ __launch_bounds__(128, 2) void rd_patch_mixed_kernel(PatchArgs quad, 
 }
 
 template <int SC>
+__global__ __launch_bounds__(128, 2) void rd_patch_mixed_batch_kernel(const PatchArgs *__restrict__ args,
+                                                                      const uint32_t *__restrict__ first, int count,
+                                                                      uint32_t nq, uint32_t nt, WeakRange weak,
+                                                                      uint32_t weak_groups)
+{
+  extern __shared__ double lds[];
+  uint32_t g = blockIdx.x;
+  if (g >= nq + nt) {
+    const uint32_t w = (g - nq - nt) * (blockDim.x / WEAK_THREADS) + threadIdx.x / WEAK_THREADS;
+    if (w < weak_groups) weak_group<PH_EULER2D, 2>(weak, w, threadIdx.x % WEAK_THREADS);
+    return;
+  }
+  const bool is_tri = g >= nq;
+  g = is_tri ? xcd_block_index(g - nq, nt) : xcd_block_index(g, nq);
+  if (is_tri) {
+    first += count + 1;
+    args += count;
+  }
+  int i = 0;
+  while (i + 1 < count && first[i + 1] <= g) ++i;
+  if (is_tri)
+    patch_body<2, 3, 3, 6, 6, true, PH_EULER2D, SC, 0>(args[i], g - first[i], lds);
+  else
+    patch_body<2, 4, 4, 9, 8, false, PH_EULER2D, SC, 0>(args[i], g - first[i], lds);
+}
+
+template <int SC>
+hipError_t launch_patch_mixed_batch(const PatchArgs *args, const uint32_t *first, int count, unsigned nq, unsigned nt,
+                                    const WeakRange &weak, unsigned weak_groups, int cells, size_t lds, hipStream_t s)
+{
+  const unsigned waves = cells / WEAK_THREADS;
+  const unsigned grid = nq + nt + (weak_groups + waves - 1) / waves;
+  hipLaunchKernelGGL((rd_patch_mixed_batch_kernel<SC>), dim3(grid), dim3(cells), lds, s, args, first, count, nq, nt, weak,
+                     weak_groups);
+  return hipGetLastError();
+}
+
+template <int SC>
 hipError_t launch_patch_mixed(const PatchArgs &quad, const PatchArgs &tri, const WeakRange &weak, unsigned weak_groups,
                               int cells, hipStream_t s)
 {
@@ -170,7 +214,10 @@ KernelSet kernel_set()
     k.patch_lin = &launch_patch<D, NG, ND, NF, NQ, AFF, PH, SC, 4>;
     k.patch_lin_lds_bytes = &patch_lds_bytes<D, ND, NQ, AFF, PH, SC, 4>;
   }
-  if constexpr (PH == PH_EULER2D && !AFF && ND == 4 && NQ == 8) k.patch_mixed = &launch_patch_mixed<SC>;
+  if constexpr (PH == PH_EULER2D && !AFF && ND == 4 && NQ == 8) {
+    k.patch_mixed = &launch_patch_mixed<SC>;
+    k.patch_mixed_batch = &launch_patch_mixed_batch<SC>;
+  }
   if constexpr (SC == SC_LDA || SC == SC_B) {
     k.cell_nodal = &launch_cell<D, NG, ND, NF, NQ, AFF, PH, SC, 2>;
     k.patch_nodal = &launch_patch<D, NG, ND, NF, NQ, AFF, PH, SC, 2>;

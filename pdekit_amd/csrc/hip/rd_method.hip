@@ -2331,8 +2331,15 @@ int grow(T **p, size_t *cap, size_t need)
 struct BatchLaunch
 {
   pdrd::PatchBatchLauncher patch = nullptr;  // null: shared-node sums
+  // mixed meshes of one launch: arguments and prefix sums of the
+  // quadrilaterals, then of the triangles; grid counts the quadrilaterals'
+  // patches, grid_tri the triangles', weak the facets' launch (-1: none)
+  pdrd::PatchMixedBatchLauncher mixed = nullptr;
+  unsigned grid_tri = 0;
+  int weak = -1;
   int m = 0;                                 // equations (shared-node sums)
   int weak_key = -1;                         // facet kernel (weak boundary conditions)
+  bool inside = false;                       // ... run by a mixed launch
   int cells = 0;                             // threads per workgroup of a patch launch
   size_t args0 = 0, first0 = 0;              // offsets in the argument / prefix arrays
   int count = 0;
@@ -2437,10 +2444,23 @@ int enqueue_batch(pdrd_batch *b, const std::vector<BatchLaunch> &patches, const 
 {
   for (const BatchLaunch &l : patches) {
     if (l.grid == 0) continue;
+    if (l.mixed) {
+      pdrd::WeakRange w{};
+      unsigned groups = 0;
+      if (l.weak >= 0) {
+        const BatchLaunch &wl = weak[l.weak];
+        w = pdrd::WeakRange{b->d_wargs + kind * wargs_per_kind + wl.args0, b->d_first + wl.first0, wl.count};
+        groups = wl.grid;
+      }
+      HIP_CHECK(l.mixed(b->d_pargs + kind * pargs_per_kind + l.args0, b->d_first + l.first0, l.count, l.grid, l.grid_tri, w,
+                        groups, l.cells, l.lds, batch_stream(b, l.lane)));
+      continue;
+    }
     HIP_CHECK(l.patch(b->d_pargs + kind * pargs_per_kind + l.args0, b->d_first + l.first0, l.count, l.grid, l.cells,
                       l.lds, batch_stream(b, l.lane)));
   }
   for (const BatchLaunch &l : weak) {
+    if (l.inside) continue;
     if (int rc = launch_facets(l.weak_key, b->d_wargs + kind * wargs_per_kind + l.args0, b->d_first + l.first0, l.count,
                                l.grid, batch_stream(b, l.lane)))
       return rc;
@@ -2538,7 +2558,23 @@ int pdrd_batch_iterate(pdrd_batch_t b, int count, const pdrd_method_t *methods, 
   // group the blocks of all methods by kernel, in order of first appearance
   std::vector<BatchLaunch> patches;
   std::vector<std::vector<std::pair<int, size_t>>> members;  // (method, block) per launch
-  for (int i = 0; i < count; ++i)
+  std::vector<int> mixed_in(count, -1);                      // the mixed launch of a method
+  for (int i = 0; i < count; ++i) {
+    const Block *quad, *tri;
+    if (!chain[i] && mixed_launch(methods[i], &quad, &tri)) {
+      size_t g = 0;
+      while (g < patches.size() && (patches[g].mixed != quad->ks.patch_mixed_batch || patches[g].cells != quad->cells)) ++g;
+      if (g == patches.size()) {
+        BatchLaunch l;
+        l.mixed = quad->ks.patch_mixed_batch;
+        l.cells = quad->cells;
+        patches.push_back(l);
+        members.emplace_back();
+      }
+      members[g].emplace_back(i, static_cast<size_t>(quad - methods[i]->blocks.data()));
+      mixed_in[i] = static_cast<int>(g);
+      continue;
+    }
     for (size_t k = 0; k < methods[i]->blocks.size(); ++k) {
       const Block &bl = methods[i]->blocks[k];
       // the kernel of the method's inputs: plain, with a nodal input, or with a source field
@@ -2558,14 +2594,15 @@ int pdrd_batch_iterate(pdrd_batch_t b, int count, const pdrd_method_t *methods, 
       }
       members[g].emplace_back(i, k);
     }
+  }
   // the streams (one for a captured graph)
   std::vector<std::vector<size_t>> kernel_of(count);
   std::vector<double> work(count, 0.0);
   for (size_t g = 0; g < patches.size(); ++g)
     for (const auto &mk : members[g]) {
-      const Block &bl = methods[mk.first]->blocks[mk.second];
       kernel_of[mk.first].push_back(g);
-      work[mk.first] += static_cast<double>(bl.ne) * bl.fe.nq * bl.fe.nd * methods[mk.first]->m;
+      for (const Block &bl : methods[mk.first]->blocks)
+        work[mk.first] += static_cast<double>(bl.ne) * bl.fe.nq * bl.fe.nd * methods[mk.first]->m;
     }
   const std::vector<int> lane = batch_lanes(kernel_of, work, b->graphs ? 1 : pdrd_batch::kStreams);
   for (size_t g = 0; g < patches.size(); ++g) patches[g].lane = lane[members[g].front().first];
@@ -2585,6 +2622,26 @@ int pdrd_batch_iterate(pdrd_batch_t b, int count, const pdrd_method_t *methods, 
     l.count = static_cast<int>(members[g].size());
     uint32_t acc = 0;
     first.push_back(0);
+    if (l.mixed) {
+      // the quadrilaterals of every member, then their triangles
+      for (int side = 0; side < 2; ++side) {
+        if (side) first.push_back(0);
+        acc = 0;
+        for (const auto &mk : members[g]) {
+          const pdrd_method *h = methods[mk.first];
+          const Block &bl = h->blocks[side ? 1 - mk.second : mk.second];
+          for (int k = 0; k < BK_COUNT; ++k) {
+            const KindPlace kp = kind_place(k, false);
+            pk[k].push_back(patch_args(h, &bl, 1, kp.outputs, excl, cfl[mk.first], kp.c));
+          }
+          l.lds = std::max(l.lds, input_lds_bytes(h, bl));
+          acc += bl.np;
+          first.push_back(acc);
+        }
+        (side ? l.grid_tri : l.grid) = acc;
+      }
+      continue;
+    }
     for (const auto &mk : members[g]) {
       pdrd_method *h = methods[mk.first];
       const Block &bl = h->blocks[mk.second];
@@ -2612,11 +2669,18 @@ int pdrd_batch_iterate(pdrd_batch_t b, int count, const pdrd_method_t *methods, 
         if (w.nf == 0) continue;
         const int key = weak_key(methods[i]->physics, w.nfn);
         size_t g = 0;
-        while (g < weak.size() && (weak[g].weak_key != key || weak[g].lane != lane[i])) ++g;
+        const bool inside = mixed_in[i] >= 0;
+        auto same = [&](const BatchLaunch &l) {
+          return inside ? static_cast<int>(&l - weak.data()) == patches[mixed_in[i]].weak
+                        : !l.inside && l.weak_key == key && l.lane == lane[i];
+        };
+        while (g < weak.size() && !same(weak[g])) ++g;
         if (g == weak.size()) {
           BatchLaunch l;
           l.weak_key = key;
           l.lane = lane[i];
+          l.inside = inside;
+          if (inside) patches[mixed_in[i]].weak = static_cast<int>(g);
           weak.push_back(l);
           wmembers.emplace_back();
         }
