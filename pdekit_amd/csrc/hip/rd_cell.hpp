@@ -1359,7 +1359,7 @@ struct PatchArgs
   int *__restrict__ status;
   uint32_t ne, np, first_patch;             // first_patch: offset of this block's patches
   int maxl;                                 // LDS rows of node state
-  int update;                               // 0: assemble (res, ws), 1: iterate
+  int update;                               // 0: assemble (res, ws), 1: iterate, 2: assemble with dt
   int outputs;                              // iterate: also store res, dt, ws and norm partials
   int excl;                                 // norm without Dirichlet rows
   double cfl;
@@ -1447,7 +1447,7 @@ template <int M>
 __device__ __forceinline__ void finish_node(const PatchArgs &a, uint32_t g, const double *acc, const double *u_old,
                                             double v, int di, double (&sq)[M + 1])
 {
-  if (a.update) {
+  if (a.update == 1) {
     double r[M], un[M], d;
     node_step<M>(a, g, acc, u_old, v, di, r, un, d);
     const bool count = a.outputs && !(a.excl && di >= 0);
@@ -1464,10 +1464,11 @@ __device__ __forceinline__ void finish_node(const PatchArgs &a, uint32_t g, cons
       a.ws[g] = acc[M];
     }
   } else {
-    const double iv = 1.0 / v;
+    const double iv = recip(v);
 #pragma unroll
     for (int k = 0; k < M; ++k) a.res[static_cast<size_t>(g) * M + k] = acc[k] * iv;
     a.ws[g] = acc[M];
+    if (a.update == 2) a.dt[g] = a.cfl * v * recip(acc[M]);
   }
 }
 
@@ -1762,7 +1763,7 @@ __device__ __forceinline__ void patch_body(const PatchArgs &a, uint32_t pl, doub
     }
   }
   if (bad) atomicOr(a.status, 1);
-  if (a.update && a.outputs) block_sum_store<M>(sq, work, a.norm_partial + static_cast<size_t>(p) * (M + 1));
+  if (a.update == 1 && a.outputs) block_sum_store<M>(sq, work, a.norm_partial + static_cast<size_t>(p) * (M + 1));
 }
 
 template <int D, int NG, int ND, int NF, int NQ, bool AFFINE, int PH, int SC, int PREC>
@@ -1819,7 +1820,7 @@ __device__ __forceinline__ void fixup_body(const FixupArgs &f, uint32_t lb, uint
     for (int k = 0; k < M; ++k) u_old[k] = f.pa.u[static_cast<size_t>(g) * M + k];
     finish_node<M>(f.pa, g, acc, u_old, f.pa.vol[g], f.pa.dir_index[g], sq);
   }
-  if (f.pa.update && f.pa.outputs) block_sum_store<M>(sq, red, f.norm_partial + static_cast<size_t>(lb) * (M + 1));
+  if (f.pa.update == 1 && f.pa.outputs) block_sum_store<M>(sq, red, f.norm_partial + static_cast<size_t>(lb) * (M + 1));
 }
 
 template <int M>
