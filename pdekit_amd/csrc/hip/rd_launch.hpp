@@ -80,7 +80,9 @@ struct KernelSet
 template <int D, int NG, int ND, int NF, int NQ, bool AFF, int PH, int SC, int PREC = 0>
 hipError_t launch_cell(const CellArgs &a, unsigned grid, unsigned block, hipStream_t s)
 {
-  const size_t lds = static_cast<size_t>(CellColumn<D, ND, NQ, AFF, PH>::value) * block * sizeof(double);
+  const size_t column = static_cast<size_t>(CellColumn<D, ND, NQ, AFF, PH>::value) * block * sizeof(double);
+  const size_t table = a.atomic ? NodeTable<ND, PhysTraits<PH>::M>::bytes(block) : 0;
+  const size_t lds = column > table ? column : table;
   hipLaunchKernelGGL((rd_cell_kernel<D, NG, ND, NF, NQ, AFF, PH, SC, PREC>), dim3(grid), dim3(block), lds, s, a);
   return hipGetLastError();
 }

@@ -51,20 +51,14 @@ int scratch_ptr(int dev, double **out)
   return PDRD_OK;
 }
 
-// Zeroes n doubles (a fill kernel rather than hipMemsetAsync, so the call can
-// be captured into a graph).
-__global__ void clear_kernel(double *__restrict__ p, size_t n)
-{
-  for (size_t i = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < n;
-       i += static_cast<size_t>(gridDim.x) * blockDim.x)
-    p[i] = 0.0;
-}
-
-// The device layout of the FE tables (TabOffsets in rd_cell.hpp): the packed
-// tables as pdrd_fe_fill writes them, then dVf as [nf][dim][nq], dV as
-// [nq][dim][nd], dVg as [nq][dim][ng]. One thread per output double.
-__global__ void table_layout_kernel(const double *__restrict__ t, int D, int NG, int ND, int NF, int NQ, int size,
-                                    double *__restrict__ out)
+// Sets up the scratch of a call: zeroes its n doubles at `acc` (a kernel rather
+// than hipMemsetAsync, so the call can be captured into a graph) and, in the
+// first workgroups, writes the device layout of the FE tables to `out`
+// (TabOffsets in rd_cell.hpp): the packed tables t as pdrd_fe_fill writes them,
+// then dVf as [nf][dim][nq], dV as [nq][dim][nd], dVg as [nq][dim][ng], one
+// thread per double.
+__global__ void setup_kernel(double *__restrict__ acc, size_t n, const double *__restrict__ t, int D, int NG, int ND,
+                             int NF, int NQ, int size, double *__restrict__ out)
 {
   const int o_dVg = NQ * D + NQ + NQ * NG;
   const int o_V = o_dVg + D * NQ * NG;
@@ -86,8 +80,10 @@ __global__ void table_layout_kernel(const double *__restrict__ t, int D, int NG,
     const int j = i - o_dVgT, q = j / (D * NG), xi = (j / NG) % D, g = j % NG;
     return t[o_dVg + (xi * NQ + q) * NG + g];
   };
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < dev_size) out[i] = value(i);
+  const size_t first = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+  const size_t stride = static_cast<size_t>(gridDim.x) * blockDim.x;
+  for (size_t i = first; i < static_cast<size_t>(dev_size); i += stride) out[i] = value(static_cast<int>(i));
+  for (size_t i = first; i < n; i += stride) acc[i] = 0.0;
 }
 
 // residual = acc / V, wave speed = acc_ws; the status word to the caller.
@@ -160,10 +156,9 @@ int pdrd_assemble_rhs_noalloc(int physics, int scheme, const double *params, int
   const hipStream_t s = static_cast<hipStream_t>(stream);
 
   // the previous call's accumulators and status are still in the array
-  const unsigned clear_blocks = std::min(blocks_for(acc + kStatusDoubles, 256), 2048u);
-  hipLaunchKernelGGL(clear_kernel, dim3(clear_blocks), dim3(256), 0, s, base + kTabDoubles, acc + kStatusDoubles);
-  hipLaunchKernelGGL(table_layout_kernel, dim3(blocks_for(dev_size, 256)), dim3(256), 0, s, tables, D, NG, ND, NF, NQ,
-                     static_cast<int>(size), d_tab);
+  const size_t clear = acc + kStatusDoubles;
+  hipLaunchKernelGGL(setup_kernel, dim3(std::min(blocks_for(std::max(clear, dev_size), 256), 2048u)), dim3(256), 0, s,
+                     base + kTabDoubles, clear, tables, D, NG, ND, NF, NQ, static_cast<int>(size), d_tab);
   if ((e = hipGetLastError()) != hipSuccess) return set_error(PDRD_EHIP, hipGetErrorString(e));
 
   if (ne) {
