@@ -39,8 +39,8 @@ struct KernelSet
   PatchBatchLauncher patch_nodal_batch = nullptr;
   PatchBatchLauncher patch_src_batch = nullptr;
   PatchLauncher patch_lin = nullptr;  // linear sweep of the mixed-precision form: J delta per cell
-  // first-order quadrilaterals of the 2D Euler equations: with the triangles
-  // of the same mesh and the weak facets in one launch
+  // quadrilaterals of the 2D Euler equations: with the triangles of the same
+  // mesh and the weak facets in one launch
   PatchMixedLauncher patch_mixed = nullptr;
   PatchMixedBatchLauncher patch_mixed_batch = nullptr;
   // with the nodal input of the scheme (LDA: artificial viscosity, B:
@@ -96,39 +96,66 @@ hipError_t launch_patch(const PatchArgs &a, unsigned grid, int cells, hipStream_
   return hipGetLastError();
 }
 
-// A sweep of a mixed mesh of first-order quadrilaterals and triangles of the 2D
+// A sweep of a mixed mesh of quadrilaterals and triangles of order P of the 2D
 // Euler equations in one launch: workgroups [0, quad.np) take the
 // quadrilaterals' patches, the next tri.np the triangles', the rest the weak
 // facets (64 to a wave), all of which only read the state of shared nodes. One
 // after the other, each kind fills the chip for a round or two and then drains
-// it: 65 536 + 131 072 cells LDA 30.6 + 16.8 us, and 5 us of facets.
-template <int SC>
-__global__ __launch_bounds__(128, 2) void rd_patch_mixed_kernel(PatchArgs quad, PatchArgs tri, WeakRange weak,
-                                                                uint32_t weak_groups)
+// it: 65 536 + 131 072 first-order cells LDA 30.6 + 16.8 us, and 5 us of facets,
+// 39 us together. Of second order only small meshes go together, whose waves
+// have a SIMD to themselves anyway (see the patch sizes in pdrd_initialize): in
+// one kernel the triangles run at the quadrilaterals' 1 wave per SIMD.
+template <int P, int SC>
+struct MixedPatch
+{
+  static constexpr int waves = P == 1 ? 2 : 1;
+  static constexpr int NDQ = (P + 1) * (P + 1), NFQ = (P + 2) * (P + 2), NDT = (P + 1) * (P + 2) / 2,
+                       NFT = (P + 2) * (P + 3) / 2;
+  static __device__ __forceinline__ void quad(const PatchArgs &a, uint32_t pl, double *lds)
+  {
+    patch_body<2, 4, NDQ, NFQ, 8, false, PH_EULER2D, SC, 0>(a, pl, lds);
+  }
+  static __device__ __forceinline__ void tri(const PatchArgs &a, uint32_t pl, double *lds)
+  {
+    patch_body<2, 3, NDT, NFT, 6, true, PH_EULER2D, SC, 0>(a, pl, lds);
+  }
+  // facets of workgroup g (counted behind the patches) of the launch
+  static __device__ __forceinline__ void facets(const WeakRange &weak, uint32_t weak_groups, uint32_t g)
+  {
+    const uint32_t w = g * (blockDim.x / WEAK_THREADS) + threadIdx.x / WEAK_THREADS;
+    if (w < weak_groups) weak_group<PH_EULER2D, P + 1>(weak, w, threadIdx.x % WEAK_THREADS);
+  }
+  static unsigned facet_blocks(unsigned weak_groups, int cells)
+  {
+    const unsigned n = cells / WEAK_THREADS;
+    return (weak_groups + n - 1) / n;
+  }
+};
+
+template <int P, int SC>
+__global__ __launch_bounds__(128, (MixedPatch<P, SC>::waves)) void rd_patch_mixed_kernel(PatchArgs quad, PatchArgs tri,
+                                                                                         WeakRange weak,
+                                                                                         uint32_t weak_groups)
 {
   extern __shared__ double lds[];
   const uint32_t g = blockIdx.x;
-  if (g < quad.np) {
-    patch_body<2, 4, 4, 9, 8, false, PH_EULER2D, SC, 0>(quad, xcd_block_index(g, quad.np), lds);
-  } else if (g < quad.np + tri.np) {
-    patch_body<2, 3, 3, 6, 6, true, PH_EULER2D, SC, 0>(tri, xcd_block_index(g - quad.np, tri.np), lds);
-  } else {
-    const uint32_t w = (g - quad.np - tri.np) * (blockDim.x / WEAK_THREADS) + threadIdx.x / WEAK_THREADS;
-    if (w < weak_groups) weak_group<PH_EULER2D, 2>(weak, w, threadIdx.x % WEAK_THREADS);
-  }
+  if (g < quad.np)
+    MixedPatch<P, SC>::quad(quad, xcd_block_index(g, quad.np), lds);
+  else if (g < quad.np + tri.np)
+    MixedPatch<P, SC>::tri(tri, xcd_block_index(g - quad.np, tri.np), lds);
+  else
+    MixedPatch<P, SC>::facets(weak, weak_groups, g - quad.np - tri.np);
 }
 
-template <int SC>
-__global__ __launch_bounds__(128, 2) void rd_patch_mixed_batch_kernel(const PatchArgs *__restrict__ args,
-                                                                      const uint32_t *__restrict__ first, int count,
-                                                                      uint32_t nq, uint32_t nt, WeakRange weak,
-                                                                      uint32_t weak_groups)
+template <int P, int SC>
+__global__ __launch_bounds__(128, (MixedPatch<P, SC>::waves)) void rd_patch_mixed_batch_kernel(
+    const PatchArgs *__restrict__ args, const uint32_t *__restrict__ first, int count, uint32_t nq, uint32_t nt,
+    WeakRange weak, uint32_t weak_groups)
 {
   extern __shared__ double lds[];
   uint32_t g = blockIdx.x;
   if (g >= nq + nt) {
-    const uint32_t w = (g - nq - nt) * (blockDim.x / WEAK_THREADS) + threadIdx.x / WEAK_THREADS;
-    if (w < weak_groups) weak_group<PH_EULER2D, 2>(weak, w, threadIdx.x % WEAK_THREADS);
+    MixedPatch<P, SC>::facets(weak, weak_groups, g - nq - nt);
     return;
   }
   const bool is_tri = g >= nq;
@@ -140,32 +167,31 @@ __global__ __launch_bounds__(128, 2) void rd_patch_mixed_batch_kernel(const Patc
   int i = 0;
   while (i + 1 < count && first[i + 1] <= g) ++i;
   if (is_tri)
-    patch_body<2, 3, 3, 6, 6, true, PH_EULER2D, SC, 0>(args[i], g - first[i], lds);
+    MixedPatch<P, SC>::tri(args[i], g - first[i], lds);
   else
-    patch_body<2, 4, 4, 9, 8, false, PH_EULER2D, SC, 0>(args[i], g - first[i], lds);
+    MixedPatch<P, SC>::quad(args[i], g - first[i], lds);
 }
 
-template <int SC>
+template <int P, int SC>
 hipError_t launch_patch_mixed_batch(const PatchArgs *args, const uint32_t *first, int count, unsigned nq, unsigned nt,
                                     const WeakRange &weak, unsigned weak_groups, int cells, size_t lds, hipStream_t s)
 {
-  const unsigned waves = cells / WEAK_THREADS;
-  const unsigned grid = nq + nt + (weak_groups + waves - 1) / waves;
-  hipLaunchKernelGGL((rd_patch_mixed_batch_kernel<SC>), dim3(grid), dim3(cells), lds, s, args, first, count, nq, nt, weak,
-                     weak_groups);
+  const unsigned grid = nq + nt + MixedPatch<P, SC>::facet_blocks(weak_groups, cells);
+  hipLaunchKernelGGL((rd_patch_mixed_batch_kernel<P, SC>), dim3(grid), dim3(cells), lds, s, args, first, count, nq, nt,
+                     weak, weak_groups);
   return hipGetLastError();
 }
 
-template <int SC>
+template <int P, int SC>
 hipError_t launch_patch_mixed(const PatchArgs &quad, const PatchArgs &tri, const WeakRange &weak, unsigned weak_groups,
                               int cells, hipStream_t s)
 {
-  const size_t lq = patch_lds_doubles<PatchWork<2, 4, 8, false, PH_EULER2D, SC, 0>, 0>(quad.maxl, cells);
-  const size_t lt = patch_lds_doubles<PatchWork<2, 3, 6, true, PH_EULER2D, SC, 0>, 0>(tri.maxl, cells);
-  const unsigned waves = cells / WEAK_THREADS;
-  const unsigned grid = quad.np + tri.np + (weak_groups + waves - 1) / waves;
-  hipLaunchKernelGGL((rd_patch_mixed_kernel<SC>), dim3(grid), dim3(cells), (lq > lt ? lq : lt) * sizeof(double), s, quad,
-                     tri, weak, weak_groups);
+  using MP = MixedPatch<P, SC>;
+  const size_t lq = patch_lds_doubles<PatchWork<2, MP::NDQ, 8, false, PH_EULER2D, SC, 0>, 0>(quad.maxl, cells);
+  const size_t lt = patch_lds_doubles<PatchWork<2, MP::NDT, 6, true, PH_EULER2D, SC, 0>, 0>(tri.maxl, cells);
+  const unsigned grid = quad.np + tri.np + MP::facet_blocks(weak_groups, cells);
+  hipLaunchKernelGGL((rd_patch_mixed_kernel<P, SC>), dim3(grid), dim3(cells), (lq > lt ? lq : lt) * sizeof(double), s,
+                     quad, tri, weak, weak_groups);
   return hipGetLastError();
 }
 
@@ -216,9 +242,10 @@ KernelSet kernel_set()
     k.patch_lin = &launch_patch<D, NG, ND, NF, NQ, AFF, PH, SC, 4>;
     k.patch_lin_lds_bytes = &patch_lds_bytes<D, ND, NQ, AFF, PH, SC, 4>;
   }
-  if constexpr (PH == PH_EULER2D && !AFF && ND == 4 && NQ == 8) {
-    k.patch_mixed = &launch_patch_mixed<SC>;
-    k.patch_mixed_batch = &launch_patch_mixed_batch<SC>;
+  if constexpr (PH == PH_EULER2D && !AFF && NQ == 8) {
+    constexpr int P = ND == 4 ? 1 : 2;
+    k.patch_mixed = &launch_patch_mixed<P, SC>;
+    k.patch_mixed_batch = &launch_patch_mixed_batch<P, SC>;
   }
   if constexpr (SC == SC_LDA || SC == SC_B) {
     k.cell_nodal = &launch_cell<D, NG, ND, NF, NQ, AFF, PH, SC, 2>;

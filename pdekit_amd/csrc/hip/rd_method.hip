@@ -764,8 +764,9 @@ int launch_fixup(pdrd_method *h, int update, int outputs, int excl, double cfl, 
 }
 
 // The quadrilateral and the triangle block of a method whose sweeps go in one
-// launch (KernelSet::patch_mixed): a mixed first-order mesh of the 2D Euler
-// equations without nodal inputs, both blocks with the same cells per patch,
+// launch (KernelSet::patch_mixed): a mixed mesh of the 2D Euler equations of
+// order 1 or 2 without nodal inputs, both blocks with the same cells per patch
+// (of second order only small meshes have that by default, see pdrd_initialize),
 // and no weak conditions on another kind of facet.
 bool mixed_launch(const pdrd_method *h, const Block **quad, const Block **tri)
 {
@@ -774,8 +775,10 @@ bool mixed_launch(const pdrd_method *h, const Block **quad, const Block **tri)
   *quad = a.ks.patch_mixed ? &a : &b;
   *tri = a.ks.patch_mixed ? &b : &a;
   const pdrd_fe_desc &t = (*tri)->fe;
-  return (*quad)->ks.patch_mixed && t.shape == PDRD_TRIAG && t.sol_order == 1 && t.nq == 6 && a.cells == b.cells &&
-         a.np && b.np && h->weak_launches.size() <= 1;
+  return (*quad)->ks.patch_mixed && t.shape == PDRD_TRIAG && t.sol_order == (*quad)->fe.sol_order && t.nq == 6 &&
+         a.cells == b.cells && a.cells <= 128 && a.np && b.np &&
+         (h->weak_launches.empty() ||
+          (h->weak_launches.size() == 1 && h->weak_launches[0].key == weak_key(PDRD_EULER2D, t.sol_order + 1)));
 }
 
 // The patch and facet kernels of one sweep: weak facets read the state at the
@@ -1362,6 +1365,35 @@ static std::vector<double> device_tables(const pdrd_fe_desc &fe, const std::vect
   return out;
 }
 
+// Default patch sizes that depend on the size of the mesh (pin: the kernels'
+// own), Euler equations only:
+//   * mixed second-order 2D meshes of up to kMixedSecond cells: 64 on both element
+//     types (the quadrilaterals' LDS allows no more), so that a sweep takes one
+//     launch (mixed_launch): 49 152 cells 53 -> 41 us, 110 592 cells 73 -> 66 us;
+//     from there on the triangles lose more by running at 1 wave per SIMD (150
+//     528 cells 85 us, 196 608 cells 83 -> 91 us);
+//   * first-order cells of up to kFirst2D / kFirst3D cells: 64, so that the waves
+//     spread evenly over the SIMDs: channel of 110 592 cells 32.8 -> 27.0 us,
+//     150 528 37.1 -> 34.5, 196 608 39.2 -> 40.5; tetrahedra 48 000 22.8 -> 18.7,
+//     196 608 37.1 -> 33.9, 384 000 56.8 -> 52.9, 663 552 alike.
+static constexpr size_t kMixedSecond = 114688, kFirst2D = 163840, kFirst3D = 524288;
+
+static void default_patch_sizes(const pdrd_method *h, std::vector<pdrd::PatchBlockIn> &pin)
+{
+  if (h->m == 1) return;
+  size_t cells = 0;
+  bool quad2 = false, tri2 = false;
+  for (const Block &b : h->blocks) {
+    cells += b.ne;
+    quad2 = quad2 || (b.fe.shape == PDRD_QUAD && b.fe.sol_order == 2);
+    tri2 = tri2 || (b.fe.shape == PDRD_TRIAG && b.fe.sol_order == 2);
+  }
+  const bool second = h->blocks.size() == 2 && quad2 && tri2 && cells <= kMixedSecond;
+  for (size_t i = 0; i < pin.size(); ++i)
+    if (second || (h->blocks[i].fe.sol_order == 1 && cells <= (h->dim == 2 ? kFirst2D : kFirst3D)))
+      pin[i].patch_size = std::min(pin[i].patch_size, 64);
+}
+
 int pdrd_initialize(pdrd_method_t h)
 {
   PDRD_TRY
@@ -1441,6 +1473,7 @@ int pdrd_initialize(pdrd_method_t h)
       x.patch_size = h->patch_cells ? std::min(h->patch_cells, b.ks.patch_size) : b.ks.patch_size;
       pin.push_back(x);
     }
+    if (!h->patch_cells) default_patch_sizes(h, pin);
     // boundary facets of the weak BCs; their nodes get one extra partial-sum
     // row per facet
     std::vector<pdrd::FacetSet> fsets;

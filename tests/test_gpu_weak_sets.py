@@ -78,3 +78,35 @@ def test_point_states_between_sweeps():
     assert np.array_equal(residual(m), base)
     m.destroy()
     ref.destroy()
+
+
+@pytest.mark.parametrize("scheme", [L.LDA, L.B])
+@pytest.mark.parametrize("order", [1, 2])
+def test_mixed_mesh_launches(order, scheme):
+    """Quadrilaterals, triangles and weak facets of a mixed mesh in one launch
+    (alone and in a batch) against chained sweeps, whose facets have a launch of
+    their own: the same bits. Ragged last patches of both element types; walls on
+    the triangles' side only (second order has no facets on quadrilaterals)."""
+    mesh = rectangle(37, 22, extent=(-0.5, 1.5, 0.0, 1.0), split=2, quad_rows=9, order=order, bump=(1.0, 0.1, 25.0, 0.5))
+    u = euler_state(mesh)
+    top = mesh.boundaries["ymax"]
+    half = top[mesh.node_coords[top, 0] <= mesh.node_coords[top, 0].mean()]
+
+    def method(chain):
+        m = PGRDMethodExplicit(L.EULER2D, scheme, params=(1.4, 287.05)).configure_mesh_data(mesh)
+        m.initialize_work_data(quad_order=4)
+        m.add_boundary_condition("WeakWall", "half", half)
+        m.add_boundary_condition("WeakFarfield", "top", top, values=u[0])
+        m.set_vec_function("solution", u)
+        m.set_option(L.OPT_CHAIN, chain)
+        return m
+
+    one, chained, batched, other = method(0), method(1), method(0), method(1)
+    n = [m.iterate(0.4, 4) for m in (one, chained)]
+    nb = Batch().iterate([batched, other], 0.4, 4)
+    assert np.array_equal(n[0], n[1]) and np.array_equal(n[0], nb[0]) and np.array_equal(n[0], nb[1])
+    for m in (chained, batched, other):
+        for f in ("solution", "residuals", "time_step"):
+            assert np.array_equal(m.vec_function(f), one.vec_function(f))
+    for m in (one, chained, batched, other):
+        m.destroy()
