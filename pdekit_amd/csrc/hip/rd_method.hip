@@ -1340,6 +1340,7 @@ int pdrd_add_cells(pdrd_method_t h, const pdrd_fe_desc *fe, const double *tables
 }
 
 static_assert(pdrd::LC_BITS == pdrd::LCONN_BITS, "patch connectivity layout differs between host and device");
+static_assert(pdrd::LC_BITS == pdrd::STAB_LC_BITS, "patch connectivity layout differs between the kernels");
 
 // The packed FE tables of a block followed by transposed copies of the
 // derivative tables (dVf as [nf][dim][nq], dV as [nq][dim][nd], dVg as
@@ -1973,6 +1974,31 @@ int stab_fill(pdrd_method *h, double *d, double v)
   return PDRD_OK;
 }
 
+// First or second pass of LF_Blend over the cells of a block: by patches where
+// the method has them, else by cells.
+int launch_lf(const pdrd_method *h, const Block &b, const pdrd::StabArgs &a, bool first)
+{
+  const dim3 grid(grid_for(a.ne, 256)), block(256);
+  if (h->patch_ok) {
+    pdrd::StabPatch p{};
+    p.lconn = b.d_lconn;
+    p.pnode_off = h->d_pnode_off + b.first_patch;
+    p.pnodes = h->d_pnodes;
+    p.pn_inner = h->d_pn_inner + b.first_patch;
+    const size_t lds = 2 * static_cast<size_t>(b.maxl) * sizeof(double);
+    if (first)
+      hipLaunchKernelGGL(pdrd::lf_patch_kernel<true>, dim3(b.np), dim3(b.cells), lds, h->stream, a, p, b.maxl);
+    else
+      hipLaunchKernelGGL(pdrd::lf_patch_kernel<false>, dim3(b.np), dim3(b.cells), lds, h->stream, a, p, b.maxl);
+  } else if (first) {
+    hipLaunchKernelGGL(pdrd::lf_indicator_kernel, grid, block, 0, h->stream, a);
+  } else {
+    hipLaunchKernelGGL(pdrd::lf_cell_kernel, grid, block, 0, h->stream, a);
+  }
+  HIP_CHECK(hipGetLastError());
+  return PDRD_OK;
+}
+
 // P1 / Q1 interpolation of the vertex values in `out` to the other nodes.
 int stab_interp(pdrd_method *h, double *out)
 {
@@ -2069,15 +2095,15 @@ int pdrd_compute_blending_coeff(pdrd_method_t h, int kind)
   for (Block &b : h->blocks) {
     pdrd::StabArgs a = stab_args(h, b);
     a.out = h->d_stab_tmp;
-    hipLaunchKernelGGL(pdrd::lf_indicator_kernel, dim3(grid_for(b.ne, 256)), dim3(256), 0, h->stream, a);
-    HIP_CHECK(hipGetLastError());
+    if (b.ne)
+      if (int rc = launch_lf(h, b, a, true)) return rc;
   }
   for (Block &b : h->blocks) {
     pdrd::StabArgs a = stab_args(h, b);
     a.in = h->d_stab_tmp;
     a.out = h->d_blend;
-    hipLaunchKernelGGL(pdrd::lf_cell_kernel, dim3(grid_for(b.ne, 256)), dim3(256), 0, h->stream, a);
-    HIP_CHECK(hipGetLastError());
+    if (b.ne)
+      if (int rc = launch_lf(h, b, a, false)) return rc;
   }
   if (int rc = stab_interp(h, h->d_blend)) return rc;
   if (!h->use_blend) drop_graph(h);
