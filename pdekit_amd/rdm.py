@@ -139,7 +139,7 @@ class PGRDMethodExplicit:
 
     def vec_function(self, which) -> np.ndarray:
         w = FIELDS[which] if isinstance(which, str) else which
-        a = np.zeros(self._shape(w))
+        a = np.empty(self._shape(w))
         L.check(L.lib().pdrd_get_field(self._h, w, L.ptr(a)), "pdrd_get_field")
         return a
 
@@ -266,9 +266,9 @@ class PGRDMethodExplicit:
         in mesh order): phi[ne][nd][m], jac[ne][nd*m][nd*m], wave[ne]."""
         blk = self.mesh.blocks[block]
         ne, nd = blk.sol_conn.shape
-        phi = np.zeros((ne, nd, self.neq))
-        jac = np.zeros((ne, nd * self.neq, nd * self.neq))
-        wave = np.zeros(ne)
+        phi = np.empty((ne, nd, self.neq))
+        jac = np.empty((ne, nd * self.neq, nd * self.neq))
+        wave = np.empty(ne)
         L.check(L.lib().pdrd_element_jacobians(self._h, int(block), L.ptr(phi), L.ptr(jac), L.ptr(wave)),
                 "pdrd_element_jacobians")
         return phi, jac, wave
