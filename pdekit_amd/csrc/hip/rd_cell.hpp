@@ -1580,6 +1580,12 @@ __device__ __forceinline__ void finish_node(const PatchArgs &a, uint32_t g, cons
     for (int k = 0; k < M; ++k) a.res[static_cast<size_t>(g) * M + k] = acc[k] * iv;
     a.ws[g] = acc[M];
     if (a.update == 2) a.dt[g] = a.cfl * v * recip(acc[M]);
+    // the strong Dirichlet value (nobody reads a node's state any more once it
+    // is finished)
+    if (di >= 0) {
+#pragma unroll
+      for (int k = 0; k < M; ++k) a.u[static_cast<size_t>(g) * M + k] = a.dir_vals[static_cast<size_t>(di) * M + k];
+    }
   }
 }
 
