@@ -93,9 +93,10 @@ enum pdrd_option {
                              stream; pdrd_last_timing then returns per-iteration means;
                              2: the same over the linear sweeps of the mixed form only */
   PDRD_OPT_PATCH_CELLS = 4, /* cells per patch workgroup, set before pdrd_initialize: 0 (each
-                             kernel's default: 256 scalar P1/P2, 128 otherwise), 64, 128 or
-                             256 (capped at the default); read back after pdrd_initialize
-                             it gives the largest in use */
+                             kernel's default: 256 scalar P1/P2, 128 otherwise; for the
+                             Euler equations on small meshes 64), 64, 128 or 256 (capped at
+                             the kernel's default); read back after pdrd_initialize it gives
+                             the largest in use */
   PDRD_OPT_REFRESH = 5,    /* mixed precision: every this many iterations (default 50) an FP64
                              sweep with fresh element Jacobians; 0 or 1: every sweep FP64 (the
                              plain iteration, bit for bit) */

@@ -17,8 +17,11 @@
 //     contravariant flux G_xi(f) = sum_d Jinv[d][xi] F_d(f) (affine cells);
 //   * N dissipation  sum_{m!=n} K+_n S^-1 K+_m (U_n - U_m) = K+_n (U_n - S^-1 sum_m K+_m U_m),
 //     S = sum_m K+_m, so one extra solve replaces the O(nd^2) pair loop;
-//   * S^-1 is never formed: S x = r and S y = sum K+_m U_m are solved by
-//     Gaussian elimination with partial pivoting done by predicated row swaps.
+//   * S^-1 is never formed: S x = r and S y = sum K+_m U_m are solved in the
+//     entropy and acoustic parts of K+ (EulerSum: one reciprocal and a
+//     Cholesky-like factor, no pivoting);
+//   * the element Jacobians keep the full matrices and eliminate with partial
+//     pivoting by predicated row swaps (solve_pp).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -527,10 +530,11 @@ struct EulerKU
 // Waves per SIMD the register allocation of a patch kernel must leave room
 // for: 5 for the scalar affine P1 / P2 cells (at most 96 VGPRs, measured
 // faster than 4 waves); 2 for the Euler cells of up to 4 nodes, which need at
-// most 256 registers but for the tetrahedra's blends (152 bytes of scratch per
+// most 256 registers but for the tetrahedra's blends (28 bytes of scratch per
 // lane): 1.57 M P1 tetrahedra per sweep at 1 and 2 waves: N 289 -> 223 us, PSI
-// / LDA blend 412 -> 336 us (the second wave covers the first's waits, a third
-// of its life); 2 for the schemes with one residual sum per node (LDA, N, PSI)
+// / LDA blend 412 -> 336 us, 233 us since the last node's residual comes from
+// the cell's (the second wave covers the first's waits, a third of its life);
+// 2 for the schemes with one residual sum per node (LDA, N, PSI)
 // on P2 triangles and for the LDA of P2 tetrahedra with the 4-point rule, which
 // need 256 registers or a few more, their pair sums in phases (PatchWork) so
 // that 8 waves fit the LDS too: 131 072 P2 triangles LDA 42.0 -> 33.9 us, N 45.5
@@ -1662,6 +1666,11 @@ __device__ __forceinline__ void patch_body(const PatchArgs &a, uint32_t pl, doub
   constexpr int GN = PatchNodes<M, ND, NQ, AFFINE, SC, PREC>::value;
   constexpr int GNS = GN > 0 ? GN : 1;
   constexpr bool EARLY = M == 1 ? ND != 6 : PatchMinWaves<M, ND, NQ, AFFINE, SC, PREC>::value == 1;
+  // The scalar kernels read of every node only what its kind needs (volume and
+  // Dirichlet index of the patch's own nodes; slot, rows and start state of the
+  // shared ones): 1.05 M P2 Burgers cells fetch 107 MB a chained sweep instead of
+  // 147 MB, 59.5 -> 58.3 us; on the Euler kernels the branches cost 1 to 5 %.
+  constexpr bool SPLIT = M == 1;
   uint32_t pg[GNS], psp[GNS];
   double pv[GNS];
   int pdi[GNS];
@@ -1675,9 +1684,25 @@ __device__ __forceinline__ void patch_body(const PatchArgs &a, uint32_t pl, doub
     }
 #pragma unroll
     for (int j = 0; j < GN; ++j) {
-      pv[j] = a.vol[pg[j]];
-      pdi[j] = a.dir_index[pg[j]];
-      psp[j] = a.slot_pos[s0 + min(t + j * PATCH, nl - 1)];
+      const int l = min(t + j * PATCH, nl - 1);
+      if constexpr (SPLIT) {
+        double v = 1.0;
+        int di = -1;
+        uint32_t sp = 0;
+        if (l < ninner) {
+          v = a.vol[pg[j]];
+          di = a.dir_index[pg[j]];
+        } else {
+          sp = a.slot_pos[s0 + l];
+        }
+        pv[j] = v;
+        pdi[j] = di;
+        psp[j] = sp;
+      } else {
+        pv[j] = a.vol[pg[j]];
+        pdi[j] = a.dir_index[pg[j]];
+        psp[j] = a.slot_pos[s0 + l];
+      }
     }
   };
   // state un of node l (id g) and its other inputs to LDS
@@ -1730,8 +1755,12 @@ __device__ __forceinline__ void patch_body(const PatchArgs &a, uint32_t pl, doub
 #pragma unroll
         for (int j = 0; j < GN; ++j) {
           const int l = min(tid + j * PATCH, nl - 1);
-          sid[j] = a.pn_sid[s0 + l];
-          rr[j] = a.pn_rows[s0 + l];
+          sid[j] = 0;
+          rr[j] = uint2{0, 0};
+          if (l >= ninner) {
+            sid[j] = a.pn_sid[s0 + l];
+            rr[j] = a.pn_rows[s0 + l];
+          }
         }
         double uo[GNS], row[GNS][2][M + 1], v[GNS];
         int di[GNS];
@@ -1739,8 +1768,12 @@ __device__ __forceinline__ void patch_body(const PatchArgs &a, uint32_t pl, doub
         for (int j = 0; j < GN; ++j) {
           const int l = min(tid + j * PATCH, nl - 1);
           uo[j] = *(l >= ninner ? a.base_in + sid[j] : a.u + pg[j]);
-          v[j] = a.vol[pg[j]];
-          di[j] = a.dir_index[pg[j]];
+          v[j] = 1.0;
+          di[j] = -1;
+          if (EARLY || l >= ninner) {
+            v[j] = a.vol[pg[j]];
+            di[j] = a.dir_index[pg[j]];
+          }
 #pragma unroll
           for (int t = 0; t < 2; ++t) {
 #pragma unroll
@@ -1756,7 +1789,7 @@ __device__ __forceinline__ void patch_body(const PatchArgs &a, uint32_t pl, doub
           if constexpr (EARLY) {
             pv[j] = v[j];
             pdi[j] = di[j];
-            psp[j] = a.slot_pos[s0 + min(l, nl - 1)];
+            psp[j] = l >= ninner ? a.slot_pos[s0 + min(l, nl - 1)] : 0;
           }
           if (l < nl) {
             double un[M] = {uo[j]};
