@@ -47,8 +47,10 @@ struct PhysParams
 // 1/x for |x| and 1/|x| in the normal range: the hardware reciprocal
 // estimate y (relative error below 2^-22) with the error e = 1 - x y taken out
 // to third order, y (1 + e + e^2): its truncation error e^3 is below 2^-66, so
-// the result is within an ulp or two of the IEEE quotient at a third of the
-// instructions of the IEEE division sequence. x = 0 gives NaN.
+// the result is the IEEE quotient but for 2 of 100 000 arguments, which round
+// the other way, at a third of the instructions of the IEEE division sequence.
+// x = 0 gives NaN. (A product a * recip(x) rounds twice: up to 1.5 ulp off the
+// quotient a / x.)
 __device__ __forceinline__ double recip(double x)
 {
   const double y = __builtin_amdgcn_rcp(x);
@@ -57,16 +59,19 @@ __device__ __forceinline__ double recip(double x)
 }
 
 // sqrt(x) and 1/sqrt(x) for x > 0 in the normal range, from one hardware
-// reciprocal square root estimate y with its error e = 1 - x y^2 taken out to
-// third order, y (1 + e/2 + 3 e^2 / 8) (the next term of the series, 5 e^3 /
-// 16, is below 2^-66). Replaces a square root and a division; x = 0 gives NaN
-// for both.
+// reciprocal square root estimate y (relative error below 2^-22) with its
+// error e = 1 - x y^2 (below 2^-21) taken out to third order, y (1 + e/2 +
+// 3 e^2 / 8); the next term of the series, 5 e^3 / 16, is below 2^-64, so
+// 1/sqrt(x) is within an ulp. Its product with x would be up to 1.7 ulp off the
+// square root; the correction by half the residual x - s^2 takes that to 0.5.
+// Replaces a square root and a division; x = 0 gives NaN for both.
 __device__ __forceinline__ void sqrt_rsqrt(double x, double &s, double &rs)
 {
   const double y = __builtin_amdgcn_rsq(x);
   const double e = fma(-x * y, y, 1.0);
   rs = fma(y * e, fma(0.375, e, 0.5), y);
-  s = x * rs;
+  const double g = x * rs;
+  s = fma(fma(-g, g, x), 0.5 * rs, g);
 }
 
 // Thermodynamic state at a point (Euler); inv_a = 1 / a.
