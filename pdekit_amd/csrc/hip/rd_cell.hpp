@@ -1668,15 +1668,26 @@ __device__ __forceinline__ void patch_body(const PatchArgs &a, uint32_t pl, doub
   // of them (id, volume, Dirichlet index, slot) is loaded here too where the
   // registers are free (EARLY) and arrives during the cell work, or else
   // behind the cell work, ahead of the pair sums, again all nodes together.
-  // Every kernel's sweep is 1 to 4 % shorter for it, those of the small
-  // scalar meshes 4 to 11 % (101 250 P3 triangles 22.6 -> 20.2 us).
+  // The timed sweeps are 1 to 4 % shorter for it, those of the small scalar
+  // meshes 4 to 11 % (101 250 P3 triangles N 22.6 -> 20.2 us). It costs registers:
+  // the scalar P3 cells run 3 waves per SIMD with it (B and the blend 2) and could
+  // run 4 (3) without, and are 2 to 11 % faster with it at every size (7 200 to 500
+  // 000 cells, LDA 13.5 against 14.1 us and 62.5 against 64.0). The Q2 Burgers
+  // cells, which also hold the flux loop's sums, fall from 3 waves to 2: the finish
+  // is loaded late there (LATE; not with a source field and the blending coefficient,
+  // which have 2 waves either way: 46 against 51 us). 160 000 cells, LDA, which 3
+  // waves hold at once: 42.6 -> 27.6 us (33.6 with the nodes one by one), 25 600
+  // cells 18.6 -> 17.7; with a nodal input or a source field 44.1 -> 33.3 us, and
+  // 18.3 -> 19.8 (21.5).
   constexpr int GN = PatchNodes<M, ND, NQ, AFFINE, SC, PREC>::value;
   constexpr int GNS = GN > 0 ? GN : 1;
-  constexpr bool EARLY = M == 1 ? ND != 6 : PatchMinWaves<M, ND, NQ, AFFINE, SC, PREC>::value == 1;
+  constexpr bool LATE = M == 1 && ND == 9 && PREC != 5 && !CellColumn<D, ND, NQ, AFFINE, PH>::linear_flux;
+  constexpr bool EARLY = M == 1 ? ND != 6 && !LATE : PatchMinWaves<M, ND, NQ, AFFINE, SC, PREC>::value == 1;
   // The scalar kernels read of every node only what its kind needs (volume and
   // Dirichlet index of the patch's own nodes; slot, rows and start state of the
-  // shared ones): 1.05 M P2 Burgers cells fetch 107 MB a chained sweep instead of
-  // 147 MB, 59.5 -> 58.3 us; on the Euler kernels the branches cost 1 to 5 %.
+  // shared ones): 1.05 M P2 Burgers cells fetch 107 MB a chained sweep, without
+  // these branches 147 MB, 58.3 against 59.5 us; on the Euler kernels the branches
+  // cost 1 to 5 %.
   constexpr bool SPLIT = M == 1;
   uint32_t pg[GNS], psp[GNS];
   double pv[GNS];
