@@ -1506,8 +1506,13 @@ static std::vector<double> device_tables(const pdrd_fe_desc &fe, const std::vect
 //   * first-order cells of up to kFirst2D / kFirst3D cells: 64, so that the waves
 //     spread evenly over the SIMDs: channel of 110 592 cells 32.8 -> 27.0 us,
 //     150 528 37.1 -> 34.5, 196 608 39.2 -> 40.5; tetrahedra 48 000 22.8 -> 18.7,
-//     196 608 37.1 -> 33.9, 384 000 56.8 -> 52.9, 663 552 alike.
-static constexpr size_t kMixedSecond = 114688, kFirst2D = 163840, kFirst3D = 524288;
+//     196 608 37.1 -> 33.9, 384 000 56.8 -> 52.9, 663 552 alike;
+//   * second-order triangles alone, with the schemes whose kernels run 2 waves
+//     per SIMD (LDA, N, PSI), up to kSecondTri cells, a wave for every SIMD, for the
+//     same reason: LDA of 40 000 cells 31.2 -> 26.0 us (30.1 at 1 wave), 65 536
+//     cells 32.2 -> 28.6 (31.0), 19 600 alike, 102 400 35.2 -> 36.8; N alike. The B
+//     scheme and the PSI / LDA blend, at 1 wave, lose (65 536 cells 28.7 -> 29.8).
+static constexpr size_t kMixedSecond = 114688, kFirst2D = 163840, kFirst3D = 524288, kSecondTri = 65536;
 
 static void default_patch_sizes(const pdrd_method *h, std::vector<pdrd::PatchBlockIn> &pin)
 {
@@ -1519,7 +1524,9 @@ static void default_patch_sizes(const pdrd_method *h, std::vector<pdrd::PatchBlo
     quad2 = quad2 || (b.fe.shape == PDRD_QUAD && b.fe.sol_order == 2);
     tri2 = tri2 || (b.fe.shape == PDRD_TRIAG && b.fe.sol_order == 2);
   }
-  const bool second = h->blocks.size() == 2 && quad2 && tri2 && cells <= kMixedSecond;
+  const bool one_sum = h->scheme == PDRD_LDA || h->scheme == PDRD_N || h->scheme == PDRD_PSI;
+  const bool second = (h->blocks.size() == 2 && quad2 && tri2 && cells <= kMixedSecond) ||
+                      (h->blocks.size() == 1 && tri2 && one_sum && cells <= kSecondTri);
   for (size_t i = 0; i < pin.size(); ++i)
     if (second || (h->blocks[i].fe.sol_order == 1 && cells <= (h->dim == 2 ? kFirst2D : kFirst3D)))
       pin[i].patch_size = std::min(pin[i].patch_size, 64);
