@@ -1621,8 +1621,9 @@ __device__ __forceinline__ void block_sum_store(double (&sq)[M + 1], double *red
   }
 }
 
-// One patch (local index pl of the block described by a) on one workgroup.
-template <int D, int NG, int ND, int NF, int NQ, bool AFFINE, int PH, int SC, int PREC>
+// One patch (local index pl of the block described by a) on one workgroup. BATCH: a
+// lies in device memory (the batch kernels).
+template <int D, int NG, int ND, int NF, int NQ, bool AFFINE, int PH, int SC, int PREC, bool BATCH = false>
 __device__ __forceinline__ void patch_body(const PatchArgs &a, uint32_t pl, double *lds)
 {
   constexpr int M = PhysTraits<PH>::M;
@@ -1678,10 +1679,14 @@ __device__ __forceinline__ void patch_body(const PatchArgs &a, uint32_t pl, doub
   // which have 2 waves either way: 46 against 51 us). 160 000 cells, LDA, which 3
   // waves hold at once: 42.6 -> 27.6 us (33.6 with the nodes one by one), 25 600
   // cells 18.6 -> 17.7; with a nodal input or a source field 44.1 -> 33.3 us, and
-  // 18.3 -> 19.8 (21.5).
+  // 18.3 -> 19.8 (21.5). Batches, whose
+  // arguments lie in memory, load it early: one method of 25 600 cells 26.3 against
+  // 30.3 us, four of 160 000 cells 168 us (198 with the nodes one by one); only where
+  // 3 waves hold the batch and 2 don't, the late loads win (160 000 cells in all 59.3
+  // against 50.7, 54.6 with the nodes one by one).
   constexpr int GN = PatchNodes<M, ND, NQ, AFFINE, SC, PREC>::value;
   constexpr int GNS = GN > 0 ? GN : 1;
-  constexpr bool LATE = M == 1 && ND == 9 && PREC != 5 && !CellColumn<D, ND, NQ, AFFINE, PH>::linear_flux;
+  constexpr bool LATE = !BATCH && M == 1 && ND == 9 && PREC != 5 && !CellColumn<D, ND, NQ, AFFINE, PH>::linear_flux;
   constexpr bool EARLY = M == 1 ? ND != 6 && !LATE : PatchMinWaves<M, ND, NQ, AFFINE, SC, PREC>::value == 1;
   // The scalar kernels read of every node only what its kind needs (volume and
   // Dirichlet index of the patch's own nodes; slot, rows and start state of the
@@ -2049,7 +2054,7 @@ rd_patch_batch_kernel(const PatchArgs *__restrict__ args, const uint32_t *__rest
   if (g >= first[count]) return;
   int i = 0;
   while (i + 1 < count && first[i + 1] <= g) ++i;
-  patch_body<D, NG, ND, NF, NQ, AFFINE, PH, SC, PREC>(args[i], g - first[i], lds);
+  patch_body<D, NG, ND, NF, NQ, AFFINE, PH, SC, PREC, true>(args[i], g - first[i], lds);
 }
 
 struct FixupArgs

@@ -57,10 +57,7 @@ def kernels():
 
 # physics Burgers; schemes LDA, N, B, PSI and the PSI / LDA blend; plain, nodal
 # inputs (LDA and B) and source fields
-@pytest.mark.parametrize("kernel", ["rd_patch_kernel", "rd_patch_batch_kernel"])
 @pytest.mark.parametrize("scheme,form", [(s, f) for s in range(5) for f in (0, 2, 3) if f != 2 or s in (0, 2)])
-def test_q2_burgers_runs_three_waves(kernels, kernel, scheme, form):
-    if form == 2 and "batch" in kernel:
-        pytest.skip("its argument arrays take the registers of a wave")
-    regs, scratch = kernels[f"{kernel}<2, 4, 9, 16, 8, false, 1, {scheme}, {form}>"]
+def test_q2_burgers_runs_three_waves(kernels, scheme, form):
+    regs, scratch = kernels[f"rd_patch_kernel<2, 4, 9, 16, 8, false, 1, {scheme}, {form}>"]
     assert regs <= 168 and scratch == 0
