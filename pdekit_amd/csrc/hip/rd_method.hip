@@ -5,16 +5,12 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
-#include <atomic>
 #include <cmath>
 #include <cstring>
 #include <map>
 #include <memory>
-#include <mutex>
 #include <stdexcept>
 #include <string>
-#include <system_error>
-#include <thread>
 #include <vector>
 
 #include "../../../include/pdekit_rd.h"
@@ -23,6 +19,7 @@
 #include "../host/fe_tables.hpp"
 #include "../host/mesh.hpp"
 #include "../host/patches.hpp"
+#include "host_stage.hpp"
 #include "rd_launch.hpp"
 #include "rd_stab.hpp"
 #include "rd_weakbc.hpp"
@@ -432,119 +429,49 @@ int dev_alloc(pdrd_method *h, T **p, size_t count)
   return PDRD_OK;
 }
 
-// Copies of results to the caller's (pageable) memory. Handed to the runtime
-// directly, such a copy is pinned or staged page range by page range: 64 KB in 46
-// us, 512 KB in 248 us, 3.2 MB in 213 us, and 29 MB into memory not touched before
-// in 7.6 ms, most of it page faults of the one copying thread. Here the data go
-// through a ring of pinned pieces, copied out while the next ones arrive, by up to
-// kStageThreads threads where there are several pieces: 18, 36, 130 us and 2.5 ms.
-// The ring (16 MiB) belongs to the process; it is made at the first copy, freed with
-// the last method, and used by one copy at a time: another thread's copy meanwhile
-// (or one of another device) goes to the runtime directly.
-constexpr size_t kStagePiece = size_t(1) << 20;
-constexpr int kStagePieces = 16, kStageThreads = 4;
-
-struct HostStage
+// The runtime calls of HostStage.
+struct Hip
 {
-  std::mutex mutex;
-  int users = 0;  // initialised methods
-  int device = -1;
-  char *buf = nullptr;
-  hipEvent_t ev[kStagePieces] = {nullptr};
-  void drop()
+  using Error = hipError_t;
+  using Stream = hipStream_t;
+  using Event = hipEvent_t;
+  static constexpr Error ok = hipSuccess;
+  static bool pageable(const void *p)
   {
-    if (buf) (void)hipHostFree(buf);
-    buf = nullptr;
-    for (hipEvent_t &e : ev) {
-      if (e) (void)hipEventDestroy(e);
-      e = nullptr;
-    }
-    device = -1;
-  }
-  bool ready(int dev)
-  {
-    if (buf) return device == dev;
-    bool ok = hipHostMalloc(reinterpret_cast<void **>(&buf), kStagePiece * kStagePieces, hipHostMallocDefault) == hipSuccess;
-    if (!ok) buf = nullptr;
-    for (hipEvent_t &e : ev) ok = ok && hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess;
-    if (!ok) {
-      (void)hipGetLastError();
-      drop();
-      return false;
-    }
-    device = dev;
+    hipPointerAttribute_t a;
+    if (hipPointerGetAttributes(&a, p) == hipSuccess) return a.type == hipMemoryTypeUnregistered;
+    (void)hipGetLastError();  // (a runtime that reports memory it does not know as an error)
     return true;
   }
+  static Error copy(void *dst, const void *src, size_t n, Stream s)
+  {
+    return hipMemcpyAsync(dst, src, n, hipMemcpyDeviceToHost, s);
+  }
+  static Error wait(Stream s) { return hipStreamSynchronize(s); }
+  static Error record(Event e, Stream s) { return hipEventRecord(e, s); }
+  static Error wait(Event e) { return hipEventSynchronize(e); }
+  static Error alloc(void **p, size_t n) { return hipHostMalloc(p, n, hipHostMallocDefault); }
+  static void free(void *p) { (void)hipHostFree(p); }
+  static Error create(Event *e) { return hipEventCreateWithFlags(e, hipEventDisableTiming); }
+  static void destroy(Event e) { (void)hipEventDestroy(e); }
+  static void clear_error() { (void)hipGetLastError(); }
 };
 
-HostStage g_stage;
+pdrd::HostStage<Hip> g_stage;
 
 void stage_user(pdrd_method *h, bool on)
 {
   if (h->stage_user == on) return;
   h->stage_user = on;
-  std::lock_guard<std::mutex> lock(g_stage.mutex);
-  g_stage.users += on ? 1 : -1;
-  if (g_stage.users == 0) g_stage.drop();
+  g_stage.user(on);
 }
 
 // n bytes at src (device) to dst (host), after what the method's stream holds;
 // complete on return.
 int copy_out(pdrd_method *h, void *dst, const void *src, size_t n)
 {
-  if (n == 0) return PDRD_OK;
-  std::unique_lock<std::mutex> lock(g_stage.mutex, std::try_to_lock);
-  if (!lock.owns_lock() || !g_stage.ready(h->device)) {
-    HIP_CHECK(hipMemcpyAsync(dst, src, n, hipMemcpyDeviceToHost, h->stream));
-    HIP_CHECK(hipStreamSynchronize(h->stream));
-    return PDRD_OK;
-  }
-  char *out = static_cast<char *>(dst);
-  const char *in = static_cast<const char *>(src);
-  if (n <= kStagePiece) {
-    HIP_CHECK(hipMemcpyAsync(g_stage.buf, in, n, hipMemcpyDeviceToHost, h->stream));
-    HIP_CHECK(hipStreamSynchronize(h->stream));
-    std::memcpy(out, g_stage.buf, n);
-    return PDRD_OK;
-  }
-  for (size_t o = 0; o < n; o += kStagePiece * kStagePieces) {
-    const size_t part = std::min(n - o, kStagePiece * kStagePieces);
-    const int pieces = static_cast<int>((part + kStagePiece - 1) / kStagePiece);
-    auto size = [&](int i) { return std::min(kStagePiece, part - i * kStagePiece); };
-    hipError_t e = hipSuccess;
-    int sent = 0;
-    for (; sent < pieces && e == hipSuccess; ++sent) {
-      e = hipMemcpyAsync(g_stage.buf + sent * kStagePiece, in + o + sent * kStagePiece, size(sent), hipMemcpyDeviceToHost,
-                         h->stream);
-      if (e == hipSuccess) e = hipEventRecord(g_stage.ev[sent], h->stream);
-    }
-    if (e != hipSuccess) {
-      (void)hipStreamSynchronize(h->stream);
-      return hip_fail(e, "copy to the host");
-    }
-    // each thread takes the next piece
-    std::atomic<int> next{0}, failed{hipSuccess};
-    auto work = [&]() noexcept {
-      for (int i = next++; i < pieces; i = next++) {
-        const hipError_t w = hipEventSynchronize(g_stage.ev[i]);
-        if (w != hipSuccess)
-          failed = w;
-        else
-          std::memcpy(out + o + i * kStagePiece, g_stage.buf + i * kStagePiece, size(i));
-      }
-    };
-    std::vector<std::thread> threads;
-    try {
-      threads.reserve(kStageThreads);
-      for (int t = 1; t < std::min(kStageThreads, pieces); ++t) threads.emplace_back(work);
-    } catch (const std::exception &) {
-      // (as many as there are)
-    }
-    work();
-    for (std::thread &t : threads) t.join();
-    if (failed != hipSuccess) return hip_fail(static_cast<hipError_t>(failed.load()), "copy to the host");
-  }
-  return PDRD_OK;
+  const hipError_t e = g_stage.copy(h->device, h->stream, dst, src, n);
+  return e == hipSuccess ? PDRD_OK : hip_fail(e, "copy to the host");
 }
 
 unsigned grid_for(uint32_t n, int threads) { return static_cast<unsigned>((n + threads - 1) / threads); }

@@ -1,0 +1,131 @@
+// Checks of HostStage without a device: copies are memcpy, "pinned" memory is what
+// Fake::pinned names, and calls can be told to fail.
+#include "host_stage.hpp"
+
+#include <cstdio>
+#include <cstdlib>
+#include <string>
+
+struct Fake
+{
+  using Error = int;
+  struct Handle
+  {
+    int id;
+    explicit operator bool() const { return id != 0; }
+  };
+  struct Stream
+  {
+  };
+  using Event = Handle;
+  static constexpr Error ok = 0;
+  static inline const char *pinned = nullptr;
+  static inline size_t pinned_bytes = 0;
+  static inline int allocs = 0, frees = 0, events = 0, direct = 0, staged = 0;
+  static inline char *buffer = nullptr;
+  static inline size_t buffer_bytes = 0;
+  static void reset() { allocs = frees = events = direct = staged = 0; }
+  static bool in(const void *p, const char *q, size_t n)
+  {
+    return q && static_cast<const char *>(p) >= q && static_cast<const char *>(p) < q + n;
+  }
+  static bool pageable(const void *p) { return !in(p, pinned, pinned_bytes); }
+  static Error copy(void *dst, const void *src, size_t n, Stream)
+  {
+    ++(in(dst, buffer, buffer_bytes) ? staged : direct);
+    std::memcpy(dst, src, n);
+    return ok;
+  }
+  static Error wait(Stream) { return ok; }
+  static Error record(Event, Stream) { return ok; }
+  static Error wait(Event) { return ok; }
+  static Error alloc(void **p, size_t n)
+  {
+    ++allocs;
+    *p = buffer = static_cast<char *>(std::malloc(n));
+    buffer_bytes = n;
+    return ok;
+  }
+  static void free(void *p)
+  {
+    ++frees;
+    buffer = nullptr;
+    std::free(p);
+  }
+  static Error create(Event *e)
+  {
+    ++events;
+    *e = {events};
+    return ok;
+  }
+  static void destroy(Event) { --events; }
+  static void clear_error() {}
+};
+
+using Stage = pdrd::HostStage<Fake>;
+
+#define CHECK(x)                                               \
+  do {                                                         \
+    if (!(x)) {                                                \
+      std::printf("%s:%d: %s\n", __FILE__, __LINE__, #x);      \
+      return 1;                                                \
+    }                                                          \
+  } while (0)
+
+static std::vector<char> data(size_t n)
+{
+  std::vector<char> v(n);
+  for (size_t i = 0; i < n; ++i) v[i] = static_cast<char>(i * 2654435761u >> 13);
+  return v;
+}
+
+// every size around the pieces and groups arrives, through the pieces
+static int sizes()
+{
+  Stage s;
+  s.user(true);
+  const size_t p = Stage::kPiece, g = p * Stage::kPieces;
+  for (size_t n : {size_t(0), size_t(1), p - 1, p, p + 1, 3 * p, g - 1, g, g + 1, 2 * g + 7}) {
+    const std::vector<char> a = data(n);
+    std::vector<char> b(n, 0);
+    Fake::direct = 0;
+    CHECK(s.copy(0, {}, b.data(), a.data(), n) == Fake::ok);
+    CHECK(a == b);
+  }
+  CHECK(Fake::direct == 0 && Fake::staged > 0);
+  // another device's copies go directly
+  const std::vector<char> a = data(5000);
+  std::vector<char> b(5000, 0);
+  CHECK(s.copy(1, {}, b.data(), a.data(), a.size()) == Fake::ok && a == b && Fake::direct == 1);
+  s.user(false);
+  CHECK(Fake::allocs == Fake::frees && Fake::events == 0);
+  return 0;
+}
+
+// pinned memory of the caller takes the copy directly, from any address in it
+static int pinned()
+{
+  Stage s;
+  s.user(true);
+  const size_t n = 3 * Stage::kPiece + 5;
+  const std::vector<char> a = data(n);
+  std::vector<char> b(n + 64, 0);
+  Fake::pinned = b.data();
+  Fake::pinned_bytes = b.size();
+  for (size_t off : {size_t(0), size_t(64)}) {
+    Fake::reset();
+    CHECK(s.copy(0, {}, b.data() + off, a.data(), n) == Fake::ok);
+    CHECK(std::memcmp(b.data() + off, a.data(), n) == 0);
+    CHECK(Fake::direct == 1 && Fake::staged == 0 && Fake::allocs == 0);
+  }
+  s.user(false);
+  return 0;
+}
+
+int main(int argc, char **argv)
+{
+  const std::string name = argc > 1 ? argv[1] : "";
+  if (name == "sizes") return sizes();
+  if (name == "pinned") return pinned();
+  return 2;
+}
