@@ -21,9 +21,12 @@ namespace pdrd {
 // copying thread. Here the data go through a buffer of pinned pieces in groups of
 // up to kPieces, copied out while the next pieces of the group arrive, by up to
 // kThreads threads where there are several pieces: 18, 36, 130 us and 2.5 ms.
-// The buffer (16 MiB) belongs to the process; it is made at the first copy, freed
-// with the last method, and used by one copy at a time: another thread's copy
-// meanwhile (or one of another device) goes to the runtime directly. So does a copy
+// The buffer (16 MiB) belongs to the process; it is freed with the last method, and
+// used by one copy at a time: another thread's copy meanwhile (or one of another
+// device) goes to the runtime directly. It is made at the first copy of several
+// pieces, or at the second one: making and freeing it takes 45 us (20 of them for the
+// events, made with the first copy of several pieces), which a program that reads one
+// small field of each of many short-lived methods would pay every time. So does a copy
 // to memory that the device reaches itself (pinned, managed or its own): 1 MB 28
 // against 70 us through the pieces, 17 MB 304 against 584 us.
 template <class Api>
@@ -49,7 +52,7 @@ public:
   {
     if (n == 0) return Api::ok;
     std::unique_lock<std::mutex> lock(mutex_, std::defer_lock);
-    if (!Api::pageable(dst) || !lock.try_lock() || !ready(device)) {
+    if (!Api::pageable(dst) || !lock.try_lock() || !ready(device, n > kPiece)) {
       if (lock.owns_lock()) lock.unlock();
       if (Error e = Api::copy(dst, src, n, stream)) return e;
       return Api::wait(stream);
@@ -105,19 +108,30 @@ private:
     return failed;
   }
 
-  bool ready(int device)
+  // The buffer for a copy of one piece or of several.
+  bool ready(int device, bool several)
   {
-    if (buf_) return device_ == device;
-    bool ok = Api::alloc(reinterpret_cast<void **>(&buf_), kPiece * kPieces) == Api::ok;
-    if (!ok) buf_ = nullptr;
+    if (!buf_) {
+      if (!several && !copied_) {
+        copied_ = true;
+        return false;
+      }
+      if (Api::alloc(reinterpret_cast<void **>(&buf_), kPiece * kPieces) != Api::ok) {
+        buf_ = nullptr;
+        Api::clear_error();
+        return false;
+      }
+      device_ = device;
+    }
+    if (device_ != device) return false;
+    if (!several || ev_[kPieces - 1]) return true;
+    bool ok = true;
     for (auto &e : ev_) ok = ok && Api::create(&e) == Api::ok;
     if (!ok) {
       Api::clear_error();
       drop();
-      return false;
     }
-    device_ = device;
-    return true;
+    return ok;
   }
 
   void drop()
@@ -129,11 +143,13 @@ private:
       e = {};
     }
     device_ = -1;
+    copied_ = false;
   }
 
   std::mutex mutex_;
   int users_ = 0;
   int device_ = -1;
+  bool copied_ = false;  // a copy has been seen that the buffer was not made for
   char *buf_ = nullptr;
   typename Api::Event ev_[kPieces] = {};
 };

@@ -22,6 +22,7 @@ struct Fake
   static inline const char *pinned = nullptr;
   static inline size_t pinned_bytes = 0;
   static inline int allocs = 0, frees = 0, events = 0, direct = 0, staged = 0;
+  static inline int max_allocs = 1 << 20, max_events = 1 << 20;
   static inline char *buffer = nullptr;
   static inline size_t buffer_bytes = 0;
   static void reset() { allocs = frees = events = direct = staged = 0; }
@@ -41,6 +42,7 @@ struct Fake
   static Error wait(Event) { return ok; }
   static Error alloc(void **p, size_t n)
   {
+    if (allocs >= max_allocs) return 2;
     ++allocs;
     *p = buffer = static_cast<char *>(std::malloc(n));
     buffer_bytes = n;
@@ -54,8 +56,8 @@ struct Fake
   }
   static Error create(Event *e)
   {
-    ++events;
-    *e = {events};
+    if (events >= max_events) return 2;
+    *e = {++events};
     return ok;
   }
   static void destroy(Event) { --events; }
@@ -85,6 +87,10 @@ static int sizes()
   Stage s;
   s.user(true);
   const size_t p = Stage::kPiece, g = p * Stage::kPieces;
+  {
+    char a = 1, b = 0;
+    CHECK(s.copy(0, {}, &b, &a, 1) == Fake::ok && b == 1);  // (the first small copy makes no pieces)
+  }
   for (size_t n : {size_t(0), size_t(1), p - 1, p, p + 1, 3 * p, g - 1, g, g + 1, 2 * g + 7}) {
     const std::vector<char> a = data(n);
     std::vector<char> b(n, 0);
@@ -122,10 +128,50 @@ static int pinned()
   return 0;
 }
 
+// one small copy makes no buffer, a second one does without events; a copy of several
+// pieces makes both at once; the last user takes them along
+static int made_late()
+{
+  const size_t p = Stage::kPiece;
+  const std::vector<char> a = data(3 * p);
+  std::vector<char> b(3 * p, 0);
+  Stage s;
+  for (int round = 0; round < 2; ++round) {
+    Fake::reset();
+    s.user(true);
+    CHECK(s.copy(0, {}, b.data(), a.data(), 100) == Fake::ok);
+    CHECK(Fake::allocs == 0 && Fake::events == 0 && Fake::direct == 1);
+    CHECK(s.copy(0, {}, b.data(), a.data(), 100) == Fake::ok);
+    CHECK(Fake::allocs == 1 && Fake::events == 0 && Fake::direct == 1 && Fake::staged == 1);
+    CHECK(s.copy(0, {}, b.data(), a.data(), 3 * p) == Fake::ok && a == b);
+    CHECK(Fake::allocs == 1 && Fake::events == Stage::kPieces && Fake::direct == 1);
+    s.user(false);
+    CHECK(Fake::frees == 1 && Fake::events == 0);
+  }
+  Fake::reset();
+  s.user(true);
+  CHECK(s.copy(0, {}, b.data(), a.data(), 3 * p) == Fake::ok);
+  CHECK(Fake::allocs == 1 && Fake::events == Stage::kPieces && Fake::direct == 0);
+  s.user(false);
+  // a buffer or an event that cannot be had: directly, and nothing is left over
+  for (int *limit : {&Fake::max_allocs, &Fake::max_events}) {
+    Fake::reset();
+    *limit = limit == &Fake::max_events ? 3 : 0;
+    std::fill(b.begin(), b.end(), 0);
+    s.user(true);
+    CHECK(s.copy(0, {}, b.data(), a.data(), 3 * p) == Fake::ok && a == b && Fake::direct == 1);
+    CHECK(Fake::allocs == Fake::frees && Fake::events == 0);
+    s.user(false);
+    *limit = 1 << 20;
+  }
+  return 0;
+}
+
 int main(int argc, char **argv)
 {
   const std::string name = argc > 1 ? argv[1] : "";
   if (name == "sizes") return sizes();
   if (name == "pinned") return pinned();
+  if (name == "made_late") return made_late();
   return 2;
 }
