@@ -105,6 +105,8 @@ private:
     }
     work();
     for (std::thread &t : threads) t.join();
+    // (the pieces go to the next copy: none of this one may still arrive)
+    if (failed != Api::ok) (void)Api::wait(stream);
     return failed;
   }
 

@@ -34,12 +34,18 @@ struct Fake
   static Error copy(void *dst, const void *src, size_t n, Stream)
   {
     ++(in(dst, buffer, buffer_bytes) ? staged : direct);
+    if (bad_copy-- == 0) return 3;
     std::memcpy(dst, src, n);
     return ok;
   }
-  static Error wait(Stream) { return ok; }
-  static Error record(Event, Stream) { return ok; }
-  static Error wait(Event) { return ok; }
+  static inline int bad_copy = -1, bad_record = -1, bad_event = -1, waits = 0;  // calls that fail, from 0
+  static Error wait(Stream)
+  {
+    ++waits;
+    return ok;
+  }
+  static Error record(Event, Stream) { return bad_record-- == 0 ? 5 : ok; }
+  static Error wait(Event e) { return e.id == bad_event ? 7 : ok; }
   static Error alloc(void **p, size_t n)
   {
     if (allocs >= max_allocs) return 2;
@@ -167,11 +173,33 @@ static int made_late()
   return 0;
 }
 
+// a call that fails in the middle of a group ends the copy with its error, and not
+// before the stream is empty: the pieces are the next copy's
+static int failures()
+{
+  const size_t n = 5 * Stage::kPiece;
+  const std::vector<char> a = data(n);
+  std::vector<char> b(n, 0);
+  Stage s;
+  s.user(true);
+  for (int which = 0; which < 3; ++which) {
+    Fake::waits = 0;
+    (which == 0 ? Fake::bad_copy : which == 1 ? Fake::bad_record : Fake::bad_event) = 2;
+    CHECK(s.copy(0, {}, b.data(), a.data(), n) == (which == 0 ? 3 : which == 1 ? 5 : 7));
+    CHECK(Fake::waits == 1);
+    Fake::bad_copy = Fake::bad_record = Fake::bad_event = -1;
+    CHECK(s.copy(0, {}, b.data(), a.data(), n) == Fake::ok && a == b);
+  }
+  s.user(false);
+  return 0;
+}
+
 int main(int argc, char **argv)
 {
   const std::string name = argc > 1 ? argv[1] : "";
   if (name == "sizes") return sizes();
   if (name == "pinned") return pinned();
   if (name == "made_late") return made_late();
+  if (name == "failures") return failures();
   return 2;
 }

@@ -17,7 +17,7 @@ def program(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("name", ["sizes", "pinned", "made_late"])
+@pytest.mark.parametrize("name", ["sizes", "pinned", "made_late", "failures"])
 def test_host_stage(program, name):
     out = subprocess.run([program, name], capture_output=True, text=True, timeout=60)
     assert out.returncode == 0, out.stdout + out.stderr
