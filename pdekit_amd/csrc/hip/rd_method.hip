@@ -835,12 +835,14 @@ bool mixed_launch(const pdrd_method *h, const Block **quad, const Block **tri)
 
 // The patch and facet kernels of one sweep: weak facets read the state at the
 // sweep's start, which u holds during the patch kernels unless the sweep's own
-// patches finish the previous one's shared nodes (c.pend).
-int launch_sweep_cells(pdrd_method *h, int update, int outputs, int excl, double cfl, Chain c = {}, bool lin = false)
+// patches finish the previous one's shared nodes (c.pend). patches_done: an event
+// to be recorded between them, the facets then in a launch of their own.
+int launch_sweep_cells(pdrd_method *h, int update, int outputs, int excl, double cfl, Chain c = {}, bool lin = false,
+                       hipEvent_t patches_done = nullptr)
 {
   const Block *quad, *tri;
   if (!lin && mixed_launch(h, &quad, &tri)) {
-    const bool with_weak = c.pend < 0 && !h->weak_launches.empty();
+    const bool with_weak = !patches_done && c.pend < 0 && !h->weak_launches.empty();
     pdrd::WeakRange w{};
     unsigned groups = 0;
     if (with_weak) {
@@ -851,9 +853,11 @@ int launch_sweep_cells(pdrd_method *h, int update, int outputs, int excl, double
     HIP_CHECK(quad->ks.patch_mixed(patch_args(h, quad, update, outputs, excl, cfl, c),
                                    patch_args(h, tri, update, outputs, excl, cfl, c), w, groups, quad->cells,
                                    h->stream));
-    return with_weak ? PDRD_OK : launch_weak(h, h->stream, c.write);
+    if (with_weak) return PDRD_OK;
+  } else if (int rc = launch_patch_blocks(h, update, outputs, excl, cfl, c, lin)) {
+    return rc;
   }
-  if (int rc = launch_patch_blocks(h, update, outputs, excl, cfl, c, lin)) return rc;
+  if (patches_done) HIP_CHECK(hipEventRecord(patches_done, h->stream));
   return launch_weak(h, h->stream, c.write);
 }
 
@@ -1234,8 +1238,8 @@ int end_iterations(pdrd_method *h, double *norm)
 // launched directly: replaying them from captured HIP graphs measured slower
 // on MI355X (25.6 against 11.1 us per sweep of a 32 768-cell P1 mesh, the
 // launches being dearer than the kernels). With timing on, events bracket the
-// patch and facet kernels (cell interval) and the fix-up (node interval) of
-// every sweep.
+// patch kernels (cell interval) and the facet kernels + fix-up (node interval) of
+// every sweep, for which facets that run in the patches' launch get their own.
 // Default: chained for the scalar physics (fewer launches, little shared-node
 // work per patch), not for the Euler systems, whose patches hold more shared
 // nodes of more equations, so that the deferred steps cost more in their
@@ -1280,8 +1284,7 @@ int iterate_patches(pdrd_method *h, double cfl, int n_iter, int excl, double *no
     c.record = !close;
     if (h->timing) {
       HIP_CHECK(hipEventRecord(h->ev[0], h->stream));
-      if (int rc = launch_sweep_cells(h, 1, out, excl, cfl, c, lin)) return rc;
-      HIP_CHECK(hipEventRecord(h->ev[1], h->stream));
+      if (int rc = launch_sweep_cells(h, 1, out, excl, cfl, c, lin, h->ev[1])) return rc;
       if (close)
         if (int rc = launch_fixup(h, 1, out, excl, cfl, c.write, lin)) return rc;
       HIP_CHECK(hipEventRecord(h->ev[2], h->stream));
