@@ -90,7 +90,8 @@ enum pdrd_option {
   PDRD_OPT_BLOCK = 2,     /* threads per block of the cell kernels (64, 128, 192, 256) */
   PDRD_OPT_TIMING = 3,    /* 1: pdrd_iterate runs eagerly and times the cell loop and the
                              nodal pass of every iteration with HIP events on the method's
-                             stream; pdrd_last_timing then returns per-iteration means;
+                             stream; pdrd_last_timing then returns per-iteration means
+                             (weak boundary facets count in the nodal pass);
                              2: the same over the linear sweeps of the mixed form only */
   PDRD_OPT_PATCH_CELLS = 4, /* cells per patch workgroup, set before pdrd_initialize: 0 (each
                              kernel's default: 256 scalar P1/P2, 128 otherwise; for the

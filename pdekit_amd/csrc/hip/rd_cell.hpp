@@ -541,7 +541,10 @@ struct EulerKU
 // -> 38.6 us, 0.20 M P2 tetrahedra LDA 146 -> 125 us a sweep. The others keep
 // the compiler's choice, 1 wave: at 2 the B scheme of P2 triangles takes 220
 // bytes of scratch (54 -> 60 us), Q2 quadrilaterals 312 (65 536 cells LDA 44 ->
-// 55 us), the P2 tetrahedra's N 172 (137 -> 151 us). The linear sweeps (PREC 4,
+// 55 us), the P2 tetrahedra's N 172 (137 -> 151 us). Forms with inputs that take
+// some scratch at these waves are still faster there: the P2 tetrahedra's LDA with
+// an artificial viscosity, 184 bytes at 2 waves, 144 us against 161 at 1 wave and no
+// scratch (196 608 cells), 79 against 88 us (82 944). The linear sweeps (PREC 4,
 // J delta per cell) are bound by the Jacobians' bandwidth and keep 4 waves (2
 // for blocks of more than 24 unknowns).
 template <int M, int ND, int NQ, bool AFFINE, int SC, int PREC>
@@ -1277,9 +1280,12 @@ __device__ __forceinline__ void gather_coords(const CellArgs &a, uint32_t e, dou
 }
 
 // Table of a workgroup's nodes in LDS (FP64 atomics): SLOTS entries of a node id
-// and its M + 1 sums, the entry of a node being its id modulo SLOTS. A power
-// of two, at least half the number of the workgroup's (cell, node) pairs, above
-// the number of nodes of cells in any sensible order, and at most 48 KiB.
+// and its M + 1 sums, the entry of a node being its id modulo SLOTS. A power of
+// two, at least half the number of the workgroup's (cell, node) pairs, which is
+// above the number of nodes of cells in any sensible order, but for two elements
+// where that would take more than 48 KiB: 256 P2 tetrahedra of the Euler equations
+// have 512 entries for about 770 nodes, 256 of their Q2 quadrilaterals 1 024 for
+// about 1 090, so that some of their nodes always go to global memory directly.
 template <int ND, int M>
 struct NodeTable
 {
@@ -1304,6 +1310,11 @@ struct NodeTable
 // bounds this kernel (its arithmetic is 5 us of it): 262 144 P2 Burgers cells 86
 // us with every part in global memory, 54 us with entries for a third of the
 // pairs, 44 us for two thirds.
+// The cells of a method are sorted by colour here and those of one colour share no
+// node; there the entries only put the atomics in the order of the nodes, still
+// worth 20 % (131 072 P1 cells 21 us directly, 17 us). It does not pay where few
+// workgroups hold cells in no order at all (32 768 shuffled P2 Euler triangles LDA
+// 64 us directly, 73 us).
 template <int D, int NG, int ND, int NF, int NQ, bool AFFINE, int PH, int SC, int PREC = 0>
 __global__ __launch_bounds__(256) void rd_cell_kernel(CellArgs a)
 {
@@ -1673,25 +1684,24 @@ __device__ __forceinline__ void patch_body(const PatchArgs &a, uint32_t pl, doub
   // The timed sweeps are 1 to 4 % shorter for it, those of the small scalar
   // meshes 4 to 11 % (101 250 P3 triangles N 22.6 -> 20.2 us). It costs registers:
   // the scalar P3 cells run 3 waves per SIMD with it (B and the blend 2) and could
-  // run 4 (3) without, and are 2 to 11 % faster with it at every size (7 200 to 500
+  // run 4 (3) without, and are up to 11 % faster with it at every size (7 200 to 500
   // 000 cells, LDA 13.5 against 14.1 us and 62.5 against 64.0). The Q2 Burgers
   // cells, which also hold the flux loop's sums, fall from 3 waves to 2: the finish
   // is loaded late there (LATE; not with a source field and the blending coefficient,
   // which have 2 waves either way: 46 against 51 us). 160 000 cells, LDA, which 3
   // waves hold at once: 42.6 -> 27.6 us (33.6 with the nodes one by one), 25 600
   // cells 18.6 -> 17.7; with a nodal input or a source field 44.1 -> 33.3 us, and
-  // 18.3 -> 19.8 (21.5). Batches, whose
-  // arguments lie in memory, load it early: one method of 25 600 cells 26.3 against
-  // 30.3 us, four of 160 000 cells 168 us (198 with the nodes one by one); only where
-  // 3 waves hold the batch and 2 don't, the late loads win (160 000 cells in all 59.3
-  // against 50.7, 54.6 with the nodes one by one).
+  // 18.3 -> 19.8 (21.5). Batches, whose arguments lie in memory, load it early: one
+  // method of 25 600 cells 26.3 against 30.3 us, four of 160 000 cells 168 us (198
+  // with the nodes one by one); only where 3 waves hold the batch and 2 don't, the
+  // late loads win (160 000 cells in all 59.3 against 50.7, 54.6 one by one).
   constexpr int GN = PatchNodes<M, ND, NQ, AFFINE, SC, PREC>::value;
   constexpr int GNS = GN > 0 ? GN : 1;
   constexpr bool LATE = !BATCH && M == 1 && ND == 9 && PREC != 5 && !CellColumn<D, ND, NQ, AFFINE, PH>::linear_flux;
   constexpr bool EARLY = M == 1 ? ND != 6 && !LATE : PatchMinWaves<M, ND, NQ, AFFINE, SC, PREC>::value == 1;
   // The scalar kernels read of every node only what its kind needs (volume and
   // Dirichlet index of the patch's own nodes; slot, rows and start state of the
-  // shared ones): 1.05 M P2 Burgers cells fetch 107 MB a chained sweep, without
+  // shared ones): 1.05 M P2 Burgers cells fetch 105 MB a chained sweep, without
   // these branches 147 MB, 58.3 against 59.5 us; on the Euler kernels the branches
   // cost 1 to 5 %.
   constexpr bool SPLIT = M == 1;

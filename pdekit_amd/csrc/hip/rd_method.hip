@@ -177,7 +177,7 @@ struct pdrd_method
   int chain = -1;              // PDRD_OPT_CHAIN (-1: the default of the method's kernels)
   size_t bytes = 0;
 
-  bool stage_user = false;     // counts in the copy ring's users
+  bool stage_user = false;     // counted among the users of g_stage
   double *norm_out = nullptr;  // host memory that the norm reduction writes, [kNormMaxM]
 
   hipStream_t stream = nullptr;
