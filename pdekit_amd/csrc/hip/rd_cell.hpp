@@ -1300,6 +1300,17 @@ struct NodeTable
   __host__ __device__ static constexpr size_t bytes(int block) { return slots(block) * entry; }
 };
 
+// Waves per SIMD that the registers of a cell kernel must leave room for: 2 for the
+// LDA of P2 triangles (Euler), which would take 259 registers and has 20 bytes of
+// scratch at 256: 786 432 P2 / Q2 cells by colours 479 -> 420 us, 250 000 triangles
+// with atomics 288 -> 275 us. The compiler's choice for the others (rotating P3 LDA
+// and the Q1 B scheme with a blending coefficient, 130 and 258 registers: no change).
+template <int M, int ND, int SC, int PREC>
+struct CellMinWaves
+{
+  static constexpr int value = (M == 4 && ND == 6 && SC == SC_LDA && PREC == 0) ? 2 : 1;
+};
+
 // Element-per-thread cell loop with a global scatter: FP64 atomics or, one
 // colour per launch, plain read-modify-write.
 // With atomics the workgroup first adds its cells' parts in LDS: a node's entry
@@ -1316,7 +1327,7 @@ struct NodeTable
 // workgroups hold cells in no order at all (32 768 shuffled P2 Euler triangles LDA
 // 64 us directly, 73 us).
 template <int D, int NG, int ND, int NF, int NQ, bool AFFINE, int PH, int SC, int PREC = 0>
-__global__ __launch_bounds__(256) void rd_cell_kernel(CellArgs a)
+__global__ __launch_bounds__(256, (CellMinWaves<PhysTraits<PH>::M, ND, SC, PREC>::value)) void rd_cell_kernel(CellArgs a)
 {
   constexpr int M = PhysTraits<PH>::M;
   extern __shared__ double lds[];

@@ -1,4 +1,4 @@
-"""Registers and scratch of the built patch kernels, from the notes of the library's own
+"""Registers and scratch of the built kernels, from the notes of the library's own
 code objects: variants that no timed workload runs must not lose a wave per SIMD
 unseen. 512 registers a lane hold 3 waves of up to 168 each."""
 import os
@@ -61,3 +61,8 @@ def kernels():
 def test_q2_burgers_runs_three_waves(kernels, scheme, form):
     regs, scratch = kernels[f"rd_patch_kernel<2, 4, 9, 16, 8, false, 1, {scheme}, {form}>"]
     assert regs <= 168 and scratch == 0
+
+
+def test_p2_lda_cells_run_two_waves(kernels):
+    regs, scratch = kernels["rd_cell_kernel<2, 3, 6, 10, 6, true, 2, 0, 0>"]
+    assert regs <= 256 and scratch <= 32
